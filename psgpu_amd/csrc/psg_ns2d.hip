@@ -215,7 +215,7 @@ int ns2d_nonlin(Ctx *c, int, const cpx<double> *in_dev, cpx<double> *out_dev) {
 template <typename P, int N, int TE>
 __global__ void __launch_bounds__(TE *(N / EPT))
 k2_xphys(const cpx<P> *__restrict__ in, double *__restrict__ out, long nrow, Grid g, const cpx<P> *__restrict__ tw) {
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, TE *(N / EPT));
   constexpr int TPX = N / EPT;
   const int team = threadIdx.x / TPX, j = threadIdx.x % TPX;
   const long row = (long)blockIdx.x * TE + team;
@@ -233,6 +233,7 @@ k2_xphys(const cpx<P> *__restrict__ in, double *__restrict__ out, long nrow, Gri
     }
     v[mm] = a;
   }
+  PSG_TWIDDLES_READY(P);
   fft_pencil<P, N, EPT, true>(v, lds + team * N, j, 1, 0, tw);
   if (valid) {
 #pragma unroll

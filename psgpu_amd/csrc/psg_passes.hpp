@@ -36,26 +36,43 @@ constexpr int EPT = 8;  // points per thread in every pencil transform
 // (launches add N*sizeof(cpx<P>) to the LDS size).
 // packed entry i of the stages from NS on, whose entries start at BASE:
 // stage NS (radix R) holds w^(r k N/(NS R)) at BASE + k (R-1) + r-1
-template <typename P, int N, int E, int NS, int BASE>
-__device__ __forceinline__ void stage_twiddle(const cpx<P> *__restrict__ tw, cpx<P> *lds_tw, int i) {
+template <int N, int E, int NS, int BASE> __device__ __forceinline__ int twiddle_src(int i) {
   if constexpr (NS < N) {
     constexpr int R = radix_at(N, E, NS), CNT = NS * (R - 1);
     if (i < BASE + CNT) {
       const int q = i - BASE, k = q / (R - 1), r = q % (R - 1) + 1;
-      lds_tw[i] = tw[(r * k) * (N / (NS * R))];
-    } else {
-      stage_twiddle<P, N, E, NS * R, BASE + CNT>(tw, lds_tw, i);
+      return (r * k) * (N / (NS * R));
+    }
+    return twiddle_src<N, E, NS * R, BASE + CNT>(i);
+  }
+  return 0;
+}
+// The table travels through registers: a kernel requests its share first
+// (request), then its pencil's data, and stores the share to LDS (commit) while
+// the data are still in flight.  The first Stockham stage needs no twiddles, so
+// a block waits for one memory latency instead of two in a row: 50 steps at
+// 64^3 in FP64 went from 1.90 to 1.84 ms, 40 at 512^2 from 1.77 to 1.70 ms.
+template <typename P, int N, int E, int NT> struct Twiddles {
+  static constexpr int M = tw_count(N, E), C = M > 0 ? (M + NT - 1) / NT : 1;
+  static_assert(M < N, "packed twiddles fit the reserved N entries");
+  cpx<P> r[C];
+  __device__ __forceinline__ void request(const cpx<P> *__restrict__ tw) {
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const int i = threadIdx.x + c * NT;
+      r[c] = i < M ? tw[twiddle_src<N, E, radix_at(N, E, 1), 0>(i)] : cpx<P>{0, 0};
     }
   }
-}
-template <typename P, int N, int E>
-__device__ __forceinline__ const cpx<P> *stage_twiddles(const cpx<P> *__restrict__ tw, cpx<P> *lds_tw) {
-  constexpr int M = tw_count(N, E);
-  static_assert(M < N, "packed twiddles fit the reserved N entries");
-  for (int i = threadIdx.x; i < M; i += blockDim.x) stage_twiddle<P, N, E, radix_at(N, E, 1), 0>(tw, lds_tw, i);
-  __syncthreads();
-  return lds_tw;
-}
+  __device__ __forceinline__ const cpx<P> *commit(cpx<P> *lds_tw) const {
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const int i = threadIdx.x + c * NT;
+      if (i < M) lds_tw[i] = r[c];
+    }
+    __syncthreads();
+    return lds_tw;
+  }
+};
 // XCD-aware tile order.  The dispatcher hands workgroups to the 8 XCDs round
 // robin (workgroup b runs on XCD b % 8, x fastest, then y, then z), and each
 // XCD has its own L2.  Column tiles of neighbouring kx ranges share cache lines
@@ -82,10 +99,14 @@ __device__ __forceinline__ TileId xcd_tile() {
 #ifndef PSG_DYN_SMEM
 #define PSG_DYN_SMEM(name) extern __shared__ __attribute__((aligned(16))) char name[]
 #endif
-#define PSG_LDS_TWIDDLES(P, N, E)                                       \
+// LDS of a transform kernel of NT threads and its share of the twiddles;
+// PSG_TWIDDLES_READY goes after the requests of the block's first data
+#define PSG_LDS_TWIDDLES(P, N, E, NT)                                  \
   PSG_DYN_SMEM(smem_raw);                                              \
   cpx<P> *lds = reinterpret_cast<cpx<P> *>(smem_raw) + (N);            \
-  tw = stage_twiddles<P, N, E>(tw, reinterpret_cast<cpx<P> *>(smem_raw))
+  Twiddles<P, N, E, (NT)> tws;                                         \
+  tws.request(tw)
+#define PSG_TWIDDLES_READY(P) tw = tws.commit(reinterpret_cast<cpx<P> *>(smem_raw))
 
 template <typename P> __device__ __forceinline__ cpx<P> to(cpx<double> a) { return {(P)a.x, (P)a.y}; }
 template <typename P> __device__ __forceinline__ cpx<P> to(cpx<float> a) { return {(P)a.x, (P)a.y}; }
@@ -253,7 +274,7 @@ template <typename P, int N, int T, bool BS, typename S = double, class LAY = La
 __global__ void __launch_bounds__(T *(N / EPT))
 k_zinv(const cpx<S> *__restrict__ st, long st_ms, long st_fs, cpx<P> *__restrict__ out, long out_ms, Grid g,
        const cpx<P> *__restrict__ tw, const int8_t *__restrict__ mask, int umask) {
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -279,6 +300,7 @@ k_zinv(const cpx<S> *__restrict__ st, long st_ms, long st_fs, cpx<P> *__restrict
   cpx<P> w[3][EPT];
   P lm[EPT];
   load(iky0, w, lm);
+  PSG_TWIDDLES_READY(P);
   constexpr int NFO = BS ? 6 : 3;
 #pragma unroll
   for (int r = 0; r < PIPE; r++) {
@@ -327,7 +349,7 @@ k_zinv(const cpx<S> *__restrict__ st, long st_ms, long st_fs, cpx<P> *__restrict
 template <typename P, int N, int T>
 __global__ void __launch_bounds__(T *(N / EPT))
 k_yinv(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cpx<P> *__restrict__ tw, int z0) {
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -341,6 +363,7 @@ k_yinv(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cp
     const int ky = wrapk(y, g.ny, g.kty);
     v[mm] = (valid && ky != PSG_NOK) ? ld_pass<NT<P, PASS_YINV>::ld>(&src[zoff<P>(g, ikx, ky + g.kty, z)]) : cpx<P>{0, 0};
   }
+  PSG_TWIDDLES_READY(P);
   fft_pencil<P, N, EPT, true>(v, lds, j, T, col, tw);
   if (valid) {
     cpx<P> *o = out + (long)mf * g.ysz;
@@ -353,7 +376,7 @@ k_yinv(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cp
 template <typename P, int N, int T>
 __global__ void __launch_bounds__(T *(N / EPT))
 k_yfwd(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cpx<P> *__restrict__ tw, int z0) {
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -363,6 +386,7 @@ k_yfwd(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cp
   cpx<P> v[EPT];
 #pragma unroll
   for (int mm = 0; mm < EPT; mm++) v[mm] = valid ? ld_pass<NT<P, PASS_YFWD>::ld>(&src[(long)(j + TP * mm) * g.xp]) : cpx<P>{0, 0};
+  PSG_TWIDDLES_READY(P);
   fft_pencil<P, N, EPT, false>(v, lds, j, T, col, tw);
   if (valid) {
     cpx<P> *o = out + (long)mf * g.zsz;
@@ -386,7 +410,7 @@ template <typename P, int N, int T, int FO, class UPD, bool FRONT = (FO <= 4), i
 __global__ void __launch_bounds__(T *(N / EPT))
 k_zfwd(const cpx<P> *__restrict__ in, Grid g, const cpx<P> *__restrict__ tw, UPD upd) {
   static_assert(PIPE == 1 || FRONT, "row pipelining needs front-loaded inputs");
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   constexpr int NV = FRONT ? FO : 1;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
@@ -405,6 +429,7 @@ k_zfwd(const cpx<P> *__restrict__ in, Grid g, const cpx<P> *__restrict__ tw, UPD
 #pragma unroll
     for (int f = 0; f < FO; f++) load(f, iky0, vin[f]);
   }
+  PSG_TWIDDLES_READY(P);
 #pragma unroll
   for (int r = 0; r < PIPE; r++) {
     const int iky = iky0 + r;
@@ -510,7 +535,7 @@ template <typename P, int N, int TEAMS, int FI, int FO, class PROD, int E = EPT,
 __global__ void __launch_bounds__(TEAMS *(N / E)) PSG_WAVES_PER_EU(WPE > 0 ? WPE : 1)
 k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, long nrows, Grid g,
         const cpx<P> *__restrict__ tw, PROD prod, int zs0) {
-  PSG_LDS_TWIDDLES(P, N, E);
+  PSG_LDS_TWIDDLES(P, N, E, TEAMS *(N / E));
   constexpr int TPX = N / E;
   constexpr bool WAVE = TPX <= 64;
   constexpr int PI = (FI + 1) / 2, PO = (FO + 1) / 2;
@@ -533,6 +558,10 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   constexpr int ix = xband<N>();
   const long ro = yoff<P>(g, 0, (int)y, (int)z);
   auto rowp = [&](int f) { return in + ((long)m * FI + f) * g.ysz + ro; };
+  // nine front-loaded fields leave no registers for the twiddles' trip (the
+  // FP32 256-point Boussinesq pass ran 0.5% slower with it)
+  constexpr bool TWFIRST = FI > 6;
+  if constexpr (TWFIRST) PSG_TWIDDLES_READY(P);
   cpx<P> vin[NV][E];
   if constexpr (FRONT) {
 #pragma unroll
@@ -540,6 +569,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
       XRow<P, N, E>::load(vin[p], rowp(2 * p), rowp(2 * p + 1 < FI ? 2 * p + 1 : 2 * p), 2 * p + 1 < FI, valid, j,
                           g);
   }
+  if constexpr (!TWFIRST) PSG_TWIDDLES_READY(P);
   P phys[2 * PI][E];
 #pragma unroll
   for (int p = 0; p < PI; p++) {
@@ -640,7 +670,8 @@ template <typename P, int N, int FI, int FO, class PROD, int E = EPT>
 __global__ void __launch_bounds__((xsplit_teams<FI, FO>() * (N / E)))
 k_xpass_split(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, long nrows, Grid g,
               const cpx<P> *__restrict__ tw, PROD prod) {
-  PSG_LDS_TWIDDLES(P, N, E);
+  constexpr int NTH = xsplit_teams<FI, FO>() * (N / E);
+  PSG_LDS_TWIDDLES(P, N, E, NTH);
   constexpr int TPX = N / E;
   constexpr bool WAVE = TPX <= 64;
   constexpr int PI = (FI + 1) / 2, PO = (FO + 1) / 2, NTEAM = xsplit_teams<FI, FO>();
@@ -658,6 +689,7 @@ k_xpass_split(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow
     const int p = team < PI ? team : PI - 1, fa = 2 * p, fb = 2 * p + 1;
     cpx<P> v[E];
     XRow<P, N, E>::load(v, rowp(fa), rowp(fb < FI ? fb : fa), fb < FI, valid && team < PI, j, g);
+    PSG_TWIDDLES_READY(P);
     fft_pencil<P, N, E, true, WAVE, SW>(v, tl, j, 1, 0, tw);
     if (team < PI) {
 #pragma unroll
@@ -753,7 +785,8 @@ __global__ void __launch_bounds__(T *(N / EPT))
 k2_yinv(const cpx<double> *__restrict__ st, long st_ms, cpx<P> *__restrict__ out, long out_ms, Grid g,
         const cpx<P> *__restrict__ tw, const int8_t *__restrict__ mask,
         const cpx<double> *__restrict__ st2 = nullptr) {
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
+  PSG_TWIDDLES_READY(P);
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -817,7 +850,8 @@ k2_yinv(const cpx<double> *__restrict__ st, long st_ms, cpx<P> *__restrict__ out
 template <typename P, int N, int T, class UPD, int NF = 2, int NG = 1>
 __global__ void __launch_bounds__(T *(N / EPT))
 k2_yfwd(const cpx<P> *__restrict__ in, long in_ms, Grid g, const cpx<P> *__restrict__ tw, UPD upd) {
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
+  PSG_TWIDDLES_READY(P);
   constexpr int TP = N / EPT, NFG = NF / NG;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();

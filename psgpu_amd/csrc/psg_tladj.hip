@@ -73,7 +73,7 @@ template <typename P, int N, int T>
 __global__ void __launch_bounds__(T *(N / EPT))
 k_zinv_curl(const cpx<double> *__restrict__ st, long fs, cpx<P> *__restrict__ out, Grid g,
             const cpx<P> *__restrict__ tw, const double *__restrict__ tab, double fac) {
-  PSG_LDS_TWIDDLES(P, N, EPT);
+  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -92,6 +92,7 @@ k_zinv_curl(const cpx<double> *__restrict__ st, long fs, cpx<P> *__restrict__ ou
     curl_k(kx, kyd, kzd, cpx<double>{s * a.x, s * a.y}, cpx<double>{s * b.x, s * b.y},
            cpx<double>{s * d.x, s * d.y}, w[0][mm], w[1][mm], w[2][mm]);
   }
+  PSG_TWIDDLES_READY(P);
 #pragma unroll
   for (int f = 0; f < 3; f++) {
     cpx<P> v[EPT];
