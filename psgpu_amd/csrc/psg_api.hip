@@ -612,7 +612,7 @@ int psg_create(const psg_config *cfg, psg_ctx **out) {
   g.alpha = hg.alpha; g.nkt = hg.nkt;
   g.xp = (g.iktx + 15) / 16 * 16;
   g.zsz = is2d ? 0 : (long)g.nz * g.ikty * g.xp;
-  g.ysz = (long)g.nz * g.ny * g.xp;
+  g.ysz = is2d ? (long)g.iktx * YCol::pitch(g) : (long)g.nz * g.ny * g.xp;
   g.inr = 1.0 / (double)hg.nr;
   g.kmax2 = ((double)g.kty - 0.5) * ((double)g.kty - 0.5);
   hipGetDevice(&c->device);

@@ -19,7 +19,7 @@ struct Grid {
   double alpha;
   long nkt;        // stored modes per field
   long zsz;        // per-field size of z-transformed buffers: nz*ikty*xp (2D: 0)
-  long ysz;        // per-field size of y-transformed buffers: nz*ny*xp
+  long ysz;        // per-field size of y-transformed buffers: nz*ny*xp (2D: columns of YCol)
   double inr;      // 1/NR
   double kmax2;    // (KTY-0.5)^2, only used for documentation/tests
 };

@@ -6,113 +6,230 @@
 // with N = -i(kx FFT(u w) + ky FFT(v w)) and forcing NZKX -= A at (0,+-KF);
 // off-mask modes of Z are zeroed at every stage.
 // (2D_NavierStokes/src_RK4/src_gmres/cuda.cu:44-76, kernels.h:247-435)
-// Each stage is three kernels: y-inverse from the state (fill, mask,
-// Biot-Savart), the shared x-pass, and a y-forward pass ending in the stage
-// update.
+// Each stage is two kernels: the shared x-pass, and a column pass (k2_col) that
+// transforms the products forward in y, applies the stage update and, while the
+// column is still on chip, transforms the next stage's (w, u, v) back in y.
 #include "psg_launch.hpp"
 
 namespace psg {
 
-// 2D y-pass column tiles: 4 columns per block from N = 512 on (the launches
-// have few blocks; half the LDS per block lets them spread over more CUs)
-template <int N, typename P> struct Col2 {
-  static constexpr int T = N >= 512 ? 4 : Col<N, P>::T;
-  static constexpr int THREADS = T * (N / EPT);
-};
-
+// RK4 stage update of one mode.  The stage input Z0 goes straight on to the
+// inverse transforms, so only the state and one running sum of the increments
+// are kept: (Z1 + 2 Z2) + 2 Z3, added in the order of the closing formula.
+// acc is private to the run and stored like the columns that the pass works on,
+// [m][ikx][iky].
 template <int STAGE> struct Upd2D {
-  cpx<double> *z, *z0, *zs;  // state, stage input, stage arrays Z1,Z2,Z3 ([m][3][nkt])
+  cpx<double> *z, *acc;
   long nkt;
   const int8_t *L;
   double dt, v2, famp, kf;
   const double *dtm = nullptr;   // per-member steps (batched Newton flows); dt 0 leaves a member unchanged
-  __device__ __forceinline__ void operator()(int m, long ik, int, double kx, double ky,
-                                             cpx<double> (&N)[2]) const {
-    cpx<double> *Z = z + (long)m * nkt + ik;
-    const double dt = dtm ? dtm[m] : this->dt;
-    if (L[ik] == 1) {
-      // NZK[ik] = FFT(v w), NZK[nkt+ik] = FFT(u w)
-      double NZKX = kx * N[1].y + ky * N[0].y;
-      double NZKY = -kx * N[1].x - ky * N[0].x;
-      if (kx == 0.0 && fabs(ky) == kf) NZKX += famp;
-      const double ZX = dt * NZKX, ZY = dt * NZKY;
-      cpx<double> *Z0 = z0 + (long)m * nkt + ik;
-      cpx<double> *S = zs + (long)m * 3 * nkt + ik;
-      const cpx<double> zn = *Z;
-      if constexpr (STAGE == 0 || STAGE == 1) {
-        S[STAGE * nkt] = cpx<double>{ZX, ZY};
-        *Z0 = cpx<double>{zn.x + 0.5 * ZX, zn.y + 0.5 * ZY};
-      } else if constexpr (STAGE == 2) {
-        S[2 * nkt] = cpx<double>{ZX, ZY};
-        *Z0 = cpx<double>{zn.x + ZX, zn.y + ZY};
-      } else {
-        const double wk = kx * kx + ky * ky;
-        const double damp1 = 1 - 0.5 * dt * v2 * wk;
-        const double damp2 = 1. / (1 + 0.5 * dt * v2 * wk);
-        const cpx<double> z1 = S[0], z2 = S[nkt], z3 = S[2 * nkt];
-        cpx<double> r;
-        r.x = damp2 * (damp1 * zn.x + (z1.x + 2 * z2.x + 2 * z3.x + ZX) / 6.);
-        r.y = damp2 * (damp1 * zn.y + (z1.y + 2 * z2.y + 2 * z3.y + ZY) / 6.);
-        *Z = r;
-        *Z0 = r;
-      }
+  int *cnt = nullptr;            // step counter of a recorded base, advanced by the last stage
+  struct In {
+    cpx<double> z, a;
+    bool on;
+  };
+  __device__ __forceinline__ In fetch(int m, long ik, long it) const {
+    In q{{0.0, 0.0}, {0.0, 0.0}, L[ik] == 1};
+    q.z = z[(long)m * nkt + ik];
+    if constexpr (STAGE > 0) q.a = acc[(long)m * nkt + it];
+    return q;
+  }
+  // N0 = FFT(v w)/NR, N1 = FFT(u w)/NR (the reference's NZK halves); returns Z0
+  __device__ __forceinline__ cpx<double> apply(const In &q, int m, long ik, long it, double kx, double ky,
+                                               cpx<double> N0, cpx<double> N1) const {
+    if (!q.on) {
+      if constexpr (STAGE == 3) z[(long)m * nkt + ik] = cpx<double>{0.0, 0.0};
+      return cpx<double>{0.0, 0.0};
+    }
+    const double h = dtm ? dtm[m] : dt;
+    double NZKX = kx * N1.y + ky * N0.y;
+    double NZKY = -kx * N1.x - ky * N0.x;
+    if (kx == 0.0 && fabs(ky) == kf) NZKX += famp;
+    const double ZX = h * NZKX, ZY = h * NZKY;
+    if constexpr (STAGE < 3) {
+      cpx<double> *A = acc + (long)m * nkt + it;
+      if constexpr (STAGE == 0) *A = cpx<double>{ZX, ZY};
+      else *A = cpx<double>{q.a.x + 2 * ZX, q.a.y + 2 * ZY};
+      const double f = STAGE == 2 ? 1.0 : 0.5;
+      return cpx<double>{q.z.x + f * ZX, q.z.y + f * ZY};
     } else {
-      *Z = cpx<double>{0.0, 0.0};
+      const double wk = kx * kx + ky * ky;
+      const double damp1 = 1 - 0.5 * h * v2 * wk;
+      const double damp2 = 1. / (1 + 0.5 * h * v2 * wk);
+      const cpx<double> r{damp2 * (damp1 * q.z.x + (q.a.x + ZX) / 6.), damp2 * (damp1 * q.z.y + (q.a.y + ZY) / 6.)};
+      z[(long)m * nkt + ik] = r;
+      return r;
+    }
+  }
+  __device__ __forceinline__ void once() const {
+    if constexpr (STAGE == 3) {
+      if (cnt) *cnt = *cnt + 1;
     }
   }
 };
 
-struct Upd2DStoreNL {
+// masked state L Z into the inverse transforms (setVelocity, kernels.h:112-147)
+struct Load2D {
+  const cpx<double> *z;
+  long nkt;
+  const int8_t *L;
+  struct In {
+    cpx<double> z;
+  };
+  __device__ __forceinline__ In fetch(int m, long ik, long) const {
+    return In{L[ik] ? z[(long)m * nkt + ik] : cpx<double>{0.0, 0.0}};
+  }
+  __device__ __forceinline__ cpx<double> apply(const In &q, int, long, long, double, double, cpx<double>,
+                                               cpx<double>) const {
+    return q.z;
+  }
+  __device__ __forceinline__ void once() const {}
+};
+
+// masked N + F into out (nonlinear right-hand side, no viscous term)
+struct Store2D {
   cpx<double> *out;
   long nkt;
   const int8_t *L;
   double famp, kf;
-  __device__ __forceinline__ void operator()(int m, long ik, int, double kx, double ky,
-                                             cpx<double> (&N)[2]) const {
-    double NZKX = kx * N[1].y + ky * N[0].y;
-    double NZKY = -kx * N[1].x - ky * N[0].x;
+  struct In {
+    double l;
+  };
+  __device__ __forceinline__ In fetch(int, long ik, long) const { return In{(double)L[ik]}; }
+  __device__ __forceinline__ cpx<double> apply(const In &q, int m, long ik, long, double kx, double ky,
+                                               cpx<double> N0, cpx<double> N1) const {
+    double NZKX = kx * N1.y + ky * N0.y;
+    double NZKY = -kx * N1.x - ky * N0.x;
     if (kx == 0.0 && fabs(ky) == kf) NZKX += famp;
-    const double ll = (double)L[ik];
-    out[(long)m * nkt + ik] = cpx<double>{ll * NZKX, ll * NZKY};
+    out[(long)m * nkt + ik] = cpx<double>{q.l * NZKX, q.l * NZKY};
+    return cpx<double>{0.0, 0.0};
   }
+  __device__ __forceinline__ void once() const {}
 };
 
-// masked copy Z0 = L Z (setVelocity, kernels.h:112-147)
-__global__ void k2_setz0(const cpx<double> *__restrict__ z, cpx<double> *__restrict__ z0, const int8_t *L,
-                         long nkt, long total) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
-    long ik = i % nkt;
-    z0[i] = L[ik] ? z[i] : cpx<double>{0.0, 0.0};
+// Column pass: one kx column per block, three teams of N/8 threads.
+//   FWD: teams 0 and 1 transform the products (v w) and (u w) forward in y;
+//        the block's threads update the column's modes from them
+//   INV: the updated column (or the loaded state) with the Hermitian fill of
+//        kx = 0 (in place in the reference, 2D_NavierStokes/src_RK4/kernels.h:82-96)
+//        and Biot-Savart (kernels.h:112-147): team f transforms field f of (w, u, v)
+// A 2D launch has few columns, so its time is the latency of one block, not
+// bandwidth.  With forward and inverse in one launch a stage takes two launches
+// instead of three, with a team per field the transforms of a column run side
+// by side, and everything a block reads is requested at its start.  At 512^2 in
+// FP64 it takes 8.2 us where separate y-forward and y-inverse passes took 9.3
+// and 7.6 us (a step 102 -> 69 us; at 128^2 89 -> 46 us), with 8 members 21.5 us.
+// Single columns ask for column-major buffers: from row-major products the pass
+// took 8.8 us, and 29.5 us with 8 members.
+// NG independent groups (blockIdx.y: base, perturbation) take their own update
+// and field range.
+template <int N> struct Col2 {
+  static constexpr int TP = N / EPT, THREADS = 3 * TP;
+  // twiddles and three rows; the updated column lies in the third row, whose
+  // team has no forward transform, where its FP64 modes fit (FP64 rows do: at
+  // 512 points five blocks then share a CU instead of four)
+  template <typename P> static constexpr bool alias() { return sizeof(P) == 8; }
+  template <typename P> static constexpr size_t lds() {
+    return (size_t)4 * N * sizeof(cpx<P>) + (alias<P>() ? 0 : (size_t)(2 * (N / 3) + 1) * sizeof(cpx<double>));
+  }
+};
+template <typename P, int N, bool FWD, bool INV, class UPD, int NG>
+__global__ void __launch_bounds__(Col2<N>::THREADS)
+k2_col(const cpx<P> *__restrict__ in, long in_ms, cpx<P> *__restrict__ out, long out_ms, Grid g,
+       const cpx<P> *__restrict__ tw, UPD upd0, UPD upd1) {
+  constexpr int TP = Col2<N>::TP, NT = Col2<N>::THREADS;
+  constexpr int NI = (2 * (N / 3) + 1 + NT - 1) / NT;   // modes of the column per thread
+  constexpr bool WAVE = TP <= 64;
+  constexpr int SW = row_swizzle<EPT>();
+  PSG_LDS_TWIDDLES(P, N, EPT, NT);
+  const int team = threadIdx.x / TP, j = threadIdx.x % TP;
+  const TileId tid = xcd_tile();
+  const int ikx = tid.x, grp = NG > 1 ? tid.y : 0, m = tid.z;
+  const UPD upd = NG > 1 && grp ? upd1 : upd0;
+  const double kx = (double)ikx * g.alpha;
+  cpx<P> *row = lds + team * N;
+  constexpr bool ALIAS = Col2<N>::template alias<P>();
+  cpx<double> *col = reinterpret_cast<cpx<double> *>(lds + (ALIAS ? 2 : 3) * N);
+  cpx<P> v[EPT];
+  if constexpr (FWD) {
+    const cpx<P> *src = in + (long)m * in_ms + (long)(grp * 2 + (team < 2 ? team : 0)) * g.ysz + YCol::col(g, ikx);
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) v[mm] = team < 2 ? src[j + TP * mm] : cpx<P>{0, 0};
+  }
+  typename UPD::In q[NI];
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    const int iky = threadIdx.x + i * NT, iy = iky < g.ikty ? iky : 0;
+    q[i] = upd.fetch(m, (long)iy * g.iktx + ikx, (long)ikx * g.ikty + iy);
+  }
+  PSG_TWIDDLES_READY(P);
+  if constexpr (FWD) {
+    fft_pencil<P, N, EPT, false, WAVE, SW>(v, row, j, 1, 0, tw);
+    team_sync<WAVE>();
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) row[j + TP * mm] = v[mm];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    const int iky = threadIdx.x + i * NT, ky = iky - g.kty;
+    if (iky < g.ikty) {
+      cpx<double> n0{0.0, 0.0}, n1{0.0, 0.0};
+      if constexpr (FWD) {
+        const int p = ky < 0 ? ky + N : ky;
+        const cpx<double> a = up(lds[p]), b = up(lds[N + p]);
+        n0 = cpx<double>{a.x * g.inr, a.y * g.inr};
+        n1 = cpx<double>{b.x * g.inr, b.y * g.inr};
+      }
+      const cpx<double> w = upd.apply(q[i], m, (long)iky * g.iktx + ikx, (long)ikx * g.ikty + iky, kx, (double)ky, n0, n1);
+      if constexpr (INV) col[iky] = w;
+    }
+  }
+  if (FWD && tid.x == 0 && tid.y == 0 && tid.z == 0 && threadIdx.x == 0) upd.once();
+  if constexpr (INV) {
+    __syncthreads();
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) {
+      const int ky = wrapk(j + TP * mm, g.ny, g.kty);
+      cpx<double> w{0.0, 0.0};
+      if (ky != PSG_NOK) {
+        const bool mirror = ikx == 0 && ky < 0;
+        w = col[(mirror ? -ky : ky) + g.kty];
+        if (mirror) w.y = -w.y;
+        if (team > 0) {
+          const double kyd = (double)ky, wk = kx * kx + kyd * kyd;
+          const double wki = 1.0 / (wk > 0.001 ? wk : 0.001);
+          w = team == 1 ? cpx<double>{-kyd * w.y * wki, kyd * w.x * wki} : cpx<double>{kx * w.y * wki, -kx * w.x * wki};
+        }
+      }
+      v[mm] = to<P>(w);
+    }
+    if constexpr (ALIAS) __syncthreads();
+    fft_pencil<P, N, EPT, true, WAVE, SW>(v, row, j, 1, 0, tw);
+    cpx<P> *o = out + (long)m * out_ms + (long)(grp * 3 + team) * g.ysz + YCol::col(g, ikx);
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) o[j + TP * mm] = v[mm];
   }
 }
 
-template <typename P> static int launch_yinv2(Ctx *c, const cpx<double> *st, cpx<P> *out, int nm) {
+// members (and NG groups) of one column pass; in: 2 NG fields, out: 3 NG fields a member
+template <typename P, bool FWD, bool INV, class UPD, int NG = 1>
+static int launch_col2(Ctx *c, const cpx<P> *in, cpx<P> *out, int nm, UPD u0, UPD u1) {
   const Grid &g = c->g;
   PSG_DISPATCH_N(g.ny, {
-    constexpr int T = Col2<N, P>::T;
-    dim3 grid((g.iktx + T - 1) / T, 3, nm);
-    size_t lds = (size_t)(N * T + N) * sizeof(cpx<P>);
-    auto k = k2_yinv<P, N, T, 1, true>;
+    const size_t lds = Col2<N>::template lds<P>();
+    auto k = k2_col<P, N, FWD, INV, UPD, NG>;
     PSG_HIP(lds_attr(k, lds));
-    hipLaunchKernelGGL(k, grid, dim3(Col2<N, P>::THREADS), lds, c->stream, st, g.nkt, out, 3 * g.ysz, g,
-                       twp<P>(c, 1), c->mask, (const cpx<double> *)nullptr);
+    hipLaunchKernelGGL(k, dim3(g.iktx, NG, nm), dim3(Col2<N>::THREADS), lds, c->stream, in, 2 * NG * g.ysz, out,
+                       3 * NG * g.ysz, g, twp<P>(c, 1), u0, u1);
   });
   PSG_HIP(hipGetLastError());
   return 0;
 }
-
-template <typename P, class UPD> static int launch_yfwd2(Ctx *c, const cpx<P> *in, UPD upd, int nm) {
-  const Grid &g = c->g;
-  PSG_DISPATCH_N(g.ny, {
-    constexpr int T = Col2<N, P>::T;
-    dim3 grid((g.iktx + T - 1) / T, 1, nm);
-    size_t lds = (size_t)(N * T + N) * sizeof(cpx<P>);
-    auto k = k2_yfwd<P, N, T, UPD>;
-    PSG_HIP(lds_attr(k, lds));
-    hipLaunchKernelGGL(k, grid, dim3(Col2<N, P>::THREADS), lds, c->stream, in, 2 * g.ysz, g, twp<P>(c, 1), upd);
-  });
-  PSG_HIP(hipGetLastError());
-  return 0;
+template <typename P, bool FWD, bool INV, class UPD>
+static int launch_col2(Ctx *c, const cpx<P> *in, cpx<P> *out, int nm, UPD u) {
+  return launch_col2<P, FWD, INV, UPD, 1>(c, in, out, nm, u, u);
 }
 
 template <typename P, int FI, int FO, class PROD>
@@ -141,7 +258,7 @@ static int launch_xpass2(Ctx *c, const cpx<P> *in, cpx<P> *out, long nrow_m, int
       constexpr int TE = Row<N>::TEAMS;
       dim3 grid((unsigned)((nrows + TE - 1) / TE));
       size_t lds = (size_t)(row_len<N>() * TE + N) * sizeof(cpx<P>);
-      auto k = k_xpass<P, N, TE, FI, FO, PROD>;
+      auto k = k_xpass<P, N, TE, FI, FO, PROD, EPT, true, false, 0, YCol>;
       PSG_HIP(lds_attr(k, lds));
       hipLaunchKernelGGL(k, grid, dim3(Row<N>::THREADS), lds, c->stream, in, out, nrow_m, nrows, g,
                          twp<P>(c, 0), prod, 0);
@@ -157,42 +274,40 @@ static int launch_xpass2(Ctx *c, const cpx<P> *in, cpx<P> *out, long nrow_m, int
     if (r_) return r_;  \
   } while (0)
 
-template <typename P, class UPD> static int rhs2(Ctx *c, const cpx<double> *z0, UPD upd, int nm) {
+static double famp2(const Ctx *c) { return c->cfg.force == PSG_FORCE_NONE ? 0.0 : c->cfg.ampfor; }
+// stage update of the context's state; of the perturbation (no forcing)
+template <int S> static Upd2D<S> upd2(const Ctx *c, int *cnt = nullptr) {
+  return Upd2D<S>{c->state, c->rh, c->g.nkt, c->mask, c->cfg.dt, c->cfg.v2, famp2(c), c->cfg.kf, c->dtm_on ? c->dtm : nullptr,
+                  cnt};
+}
+template <int S> static Upd2D<S> pert2(const Ctx *c, int *cnt = nullptr) {
+  return Upd2D<S>{c->tl_state, c->tl_rh, c->g.nkt, c->mask, c->cfg.dt, c->cfg.v2, 0.0, c->cfg.kf, nullptr, cnt};
+}
+static Load2D load2(const Ctx *c, const cpx<double> *z) { return Load2D{z, c->g.nkt, c->mask}; }
+
+// one stage from the y-space fields in B, which it leaves ready for the next
+template <typename P, class UPD> static int stage2(Ctx *c, UPD upd, int nm) {
   const Grid &g = c->g;
   cpx<P> *B = (cpx<P> *)c->bufB, *Cb = (cpx<P> *)c->bufC;
   const long Y = (long)g.iktx * g.ny;
   const size_t b = sizeof(cpx<P>);
-  prof_begin(c, "yinv2", (long)(g.nkt * 16 + 3 * Y * b) * nm);
-  PSG_TRY2(launch_yinv2<P>(c, z0, B, nm));
-  prof_end(c);
   prof_begin(c, "xpass2", (long)(5 * Y * b) * nm);
   PSG_TRY2((launch_xpass2<P, 3, 2>(c, B, Cb, g.ny, nm, Prod2D<P>{})));
   prof_end(c);
-  prof_begin(c, "yfwd2_update", (long)(2 * Y * b + 4 * g.nkt * 16) * nm);
-  PSG_TRY2((launch_yfwd2<P>(c, Cb, upd, nm)));
+  prof_begin(c, "ycol2_update", (long)(5 * Y * b + 3 * g.nkt * 16) * nm);
+  PSG_TRY2((launch_col2<P, true, true>(c, Cb, B, nm, upd)));
   prof_end(c);
   return 0;
 }
 
 template <typename P> static int run2_t(Ctx *c, int nsteps, bool first) {
-  const Grid &g = c->g;
-  const long total = g.nkt * c->batch;
-  if (first) {
-    // stage input Z0 = masked state; later steps leave Z0 = state themselves
-    hipLaunchKernelGGL(k2_setz0, dim3((unsigned)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096)),
-                       dim3(256), 0, c->stream, c->state, c->stage, c->mask, g.nkt, total);
-    PSG_HIP(hipGetLastError());
-  }
-  const double famp = c->cfg.force == PSG_FORCE_NONE ? 0.0 : c->cfg.ampfor;
+  // a run starts from the masked state; every later stage finds its fields in B
+  if (first) PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, (cpx<P> *)c->bufB, c->batch, load2(c, c->state))));
   for (int nt = 0; nt < nsteps; nt++) {
-    Upd2D<0> u0{c->state, c->stage, c->rh, g.nkt, c->mask, c->cfg.dt, c->cfg.v2, famp, c->cfg.kf, c->dtm_on ? c->dtm : nullptr};
-    PSG_TRY2(rhs2<P>(c, c->stage, u0, c->batch));
-    Upd2D<1> u1{c->state, c->stage, c->rh, g.nkt, c->mask, c->cfg.dt, c->cfg.v2, famp, c->cfg.kf, c->dtm_on ? c->dtm : nullptr};
-    PSG_TRY2(rhs2<P>(c, c->stage, u1, c->batch));
-    Upd2D<2> u2{c->state, c->stage, c->rh, g.nkt, c->mask, c->cfg.dt, c->cfg.v2, famp, c->cfg.kf, c->dtm_on ? c->dtm : nullptr};
-    PSG_TRY2(rhs2<P>(c, c->stage, u2, c->batch));
-    Upd2D<3> u3{c->state, c->stage, c->rh, g.nkt, c->mask, c->cfg.dt, c->cfg.v2, famp, c->cfg.kf, c->dtm_on ? c->dtm : nullptr};
-    PSG_TRY2(rhs2<P>(c, c->stage, u3, c->batch));
+    PSG_TRY2(stage2<P>(c, upd2<0>(c), c->batch));
+    PSG_TRY2(stage2<P>(c, upd2<1>(c), c->batch));
+    PSG_TRY2(stage2<P>(c, upd2<2>(c), c->batch));
+    PSG_TRY2(stage2<P>(c, upd2<3>(c), c->batch));
   }
   return 0;
 }
@@ -202,9 +317,10 @@ int ns2d_run(Ctx *c, int nsteps, bool first) {
 }
 
 template <typename P> static int nonlin2_t(Ctx *c, const cpx<double> *in, cpx<double> *out) {
-  const double famp = c->cfg.force == PSG_FORCE_NONE ? 0.0 : c->cfg.ampfor;
-  Upd2DStoreNL u{out, c->g.nkt, c->mask, famp, c->cfg.kf};
-  return rhs2<P>(c, in, u, 1);
+  cpx<P> *B = (cpx<P> *)c->bufB, *Cb = (cpx<P> *)c->bufC;
+  PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, B, 1, load2(c, in))));
+  PSG_TRY2((launch_xpass2<P, 3, 2>(c, B, Cb, c->g.ny, 1, Prod2D<P>{})));
+  return launch_col2<P, true, false>(c, Cb, (cpx<P> *)nullptr, 1, Store2D{out, c->g.nkt, c->mask, famp2(c), c->cfg.kf});
 }
 
 int ns2d_nonlin(Ctx *c, int, const cpx<double> *in_dev, cpx<double> *out_dev) {
@@ -221,15 +337,15 @@ k2_xphys(const cpx<P> *__restrict__ in, double *__restrict__ out, long nrow, Gri
   const long row = (long)blockIdx.x * TE + team;
   const bool valid = row < nrow;
   const int f = blockIdx.y;
-  const cpx<P> *ra = in + (long)f * g.ysz + yrow<P>(g, valid ? row : 0);
+  const cpx<P> *ra = in + (long)f * g.ysz + YCol::row(g, valid ? (int)row : 0, 0);
   cpx<P> v[EPT];
 #pragma unroll
   for (int mm = 0; mm < EPT; mm++) {
     const int k = j + TPX * mm;
     cpx<P> a{0, 0};
     if (valid) {
-      if (k < g.iktx) { a = ra[ycol<P>(g, k)]; if (k == 0) a.y = 0; }
-      else if (k > N - g.iktx) { a = ra[ycol<P>(g, N - k)]; a.y = -a.y; }
+      if (k < g.iktx) { a = ra[YCol::col(g, k)]; if (k == 0) a.y = 0; }
+      else if (k > N - g.iktx) { a = ra[YCol::col(g, N - k)]; a.y = -a.y; }
     }
     v[mm] = a;
   }
@@ -245,10 +361,7 @@ template <typename P> static int physical2_t(Ctx *c, int member, double *out) {
   const Grid &g = c->g;
   cpx<P> *B = (cpx<P> *)c->bufB;
   // physical fields of the masked state (w, u, v)
-  const long total = g.nkt;
-  hipLaunchKernelGGL(k2_setz0, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, c->stream,
-                     c->state + (long)member * g.nkt, c->tmp, c->mask, g.nkt, total);
-  PSG_TRY2(launch_yinv2<P>(c, c->tmp, B, 1));
+  PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, B, 1, load2(c, c->state + (long)member * g.nkt))));
   long nrow = g.ny;
   PSG_DISPATCH_N(g.nx, {
     constexpr int TE = Row<N>::TEAMS;
@@ -271,103 +384,25 @@ int ns2d_physical(Ctx *c, int member, double *out_dev) {
 // Base and perturbation advance together through the same RK4/CN stages:
 // the perturbation stage increments use the linearised nonlinear term
 // dN = -i(kx FFT(du w + u dw) + ky FFT(dv w + v dw)) (no forcing) with the
-// same damping factors and masks as the base update.
-template <int STAGE> struct Upd2DTL {
-  Upd2D<STAGE> base;
-  cpx<double> *dz, *dz0, *dzs;
-  __device__ __forceinline__ void operator()(int m, long ik, int i0, double kx, double ky,
-                                             cpx<double> (&N)[4]) const {
-    cpx<double> nb[2] = {N[0], N[1]}, np[2] = {N[2], N[3]};
-    base(m, ik, i0, kx, ky, nb);
-    pert(m, ik, kx, ky, np);
-  }
-  // group 0: the base update from N[0..1]; group 1: the perturbation's from N[2..3]
-  __device__ __forceinline__ void part(int grp, int m, long ik, int i0, double kx, double ky,
-                                       cpx<double> (&N)[2]) const {
-    if (grp == 0) base(m, ik, i0, kx, ky, N);
-    else pert(m, ik, kx, ky, N);
-  }
-  // N = {FFT(dv w + v dw), FFT(du w + u dw)} / NR
-  __device__ __forceinline__ void pert(int m, long ik, double kx, double ky, cpx<double> (&N)[2]) const {
-    const long nkt = base.nkt;
-    cpx<double> *Z = dz + (long)m * nkt + ik;
-    if (base.L[ik] == 1) {
-      const double NX = kx * N[1].y + ky * N[0].y;
-      const double NY = -kx * N[1].x - ky * N[0].x;
-      const double dt = base.dt;
-      const double ZX = dt * NX, ZY = dt * NY;
-      cpx<double> *Z0 = dz0 + (long)m * nkt + ik;
-      cpx<double> *S = dzs + (long)m * 3 * nkt + ik;
-      const cpx<double> zn = *Z;
-      if constexpr (STAGE == 0 || STAGE == 1) {
-        S[STAGE * nkt] = cpx<double>{ZX, ZY};
-        *Z0 = cpx<double>{zn.x + 0.5 * ZX, zn.y + 0.5 * ZY};
-      } else if constexpr (STAGE == 2) {
-        S[2 * nkt] = cpx<double>{ZX, ZY};
-        *Z0 = cpx<double>{zn.x + ZX, zn.y + ZY};
-      } else {
-        const double wk = kx * kx + ky * ky;
-        const double damp1 = 1 - 0.5 * dt * base.v2 * wk;
-        const double damp2 = 1. / (1 + 0.5 * dt * base.v2 * wk);
-        const cpx<double> z1 = S[0], z2 = S[nkt], z3 = S[2 * nkt];
-        cpx<double> r;
-        r.x = damp2 * (damp1 * zn.x + (z1.x + 2 * z2.x + 2 * z3.x + ZX) / 6.);
-        r.y = damp2 * (damp1 * zn.y + (z1.y + 2 * z2.y + 2 * z3.y + ZY) / 6.);
-        *Z = r;
-        *Z0 = r;
-      }
-    } else {
-      *Z = cpx<double>{0.0, 0.0};
-    }
-  }
-};
-
-template <typename P, class UPD> static int rhs2_tl(Ctx *c, UPD upd, int nm) {
-  const Grid &g = c->g;
+// same damping factors and masks as the base update.  The x-pass mixes them;
+// the column pass takes them as two independent groups.
+template <typename P, int S> static int stage2_tl(Ctx *c) {
   cpx<P> *B = (cpx<P> *)c->tl_bufB, *Cb = (cpx<P> *)c->tl_bufC;
-  PSG_DISPATCH_N(g.ny, {
-    constexpr int T = Col2<N, P>::T;
-    dim3 grid((g.iktx + T - 1) / T, 6, nm);
-    size_t lds = (size_t)(N * T + N) * sizeof(cpx<P>);
-    auto k = k2_yinv<P, N, T, 2, true>;
-    PSG_HIP(lds_attr(k, lds));
-    hipLaunchKernelGGL(k, grid, dim3(Col2<N, P>::THREADS), lds, c->stream, c->stage, g.nkt, B, 6 * g.ysz, g,
-                       twp<P>(c, 1), c->mask, c->tl_stage);
-  });
-  PSG_HIP(hipGetLastError());
-  PSG_TRY2((launch_xpass2<P, 6, 4>(c, B, Cb, g.ny, nm, Prod2DTL<P>{})));
-  PSG_DISPATCH_N(g.ny, {
-    constexpr int T = Col2<N, P>::T;
-    dim3 grid((g.iktx + T - 1) / T, 2, nm);
-    size_t lds = (size_t)(N * T + N) * sizeof(cpx<P>);
-    auto k = k2_yfwd<P, N, T, UPD, 4, 2>;
-    PSG_HIP(lds_attr(k, lds));
-    hipLaunchKernelGGL(k, grid, dim3(Col2<N, P>::THREADS), lds, c->stream, Cb, 4 * g.ysz, g, twp<P>(c, 1), upd);
-  });
-  PSG_HIP(hipGetLastError());
-  return 0;
+  Upd2D<S> base = upd2<S>(c);
+  base.dtm = nullptr;
+  PSG_TRY2((launch_xpass2<P, 6, 4>(c, B, Cb, c->g.ny, c->batch, Prod2DTL<P>{})));
+  return launch_col2<P, true, true, Upd2D<S>, 2>(c, Cb, B, c->batch, base, pert2<S>(c));
 }
 
 template <typename P> static int run2tl_t(Ctx *c, int nsteps, bool first) {
-  const Grid &g = c->g;
-  const long total = g.nkt * c->batch;
-  const unsigned gb = (unsigned)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-  if (first) {
-    hipLaunchKernelGGL(k2_setz0, dim3(gb), dim3(256), 0, c->stream, c->state, c->stage, c->mask, g.nkt, total);
-    hipLaunchKernelGGL(k2_setz0, dim3(gb), dim3(256), 0, c->stream, c->tl_state, c->tl_stage, c->mask, g.nkt,
-                       total);
-    PSG_HIP(hipGetLastError());
-  }
-  const double famp = c->cfg.force == PSG_FORCE_NONE ? 0.0 : c->cfg.ampfor;
+  if (first)
+    PSG_TRY2((launch_col2<P, false, true, Load2D, 2>(c, nullptr, (cpx<P> *)c->tl_bufB, c->batch, load2(c, c->state),
+                                                     load2(c, c->tl_state))));
   for (int nt = 0; nt < nsteps; nt++) {
-#define PSG_TL_STAGE(S)                                                                                    \
-    {                                                                                                      \
-      Upd2DTL<S> u{{c->state, c->stage, c->rh, g.nkt, c->mask, c->cfg.dt, c->cfg.v2, famp, c->cfg.kf},     \
-                   c->tl_state, c->tl_stage, c->tl_rh};                                                    \
-      PSG_TRY2(rhs2_tl<P>(c, u, c->batch));                                                                 \
-    }
-    PSG_TL_STAGE(0) PSG_TL_STAGE(1) PSG_TL_STAGE(2) PSG_TL_STAGE(3)
-#undef PSG_TL_STAGE
+    PSG_TRY2((stage2_tl<P, 0>(c)));
+    PSG_TRY2((stage2_tl<P, 1>(c)));
+    PSG_TRY2((stage2_tl<P, 2>(c)));
+    PSG_TRY2((stage2_tl<P, 3>(c)));
   }
   return 0;
 }
@@ -380,8 +415,8 @@ int ns2d_tl_run(Ctx *c, int nsteps, bool first) {
 // ------------------------------------------------------------------ recorded base
 // A base flow whose x-pass uses Prod2DRec stores the physical (w, u, v) of
 // every stage at slot 4*step + stage, step being the device counter that the
-// last stage's y-forward advances (StepEnd).  The perturbation-only flow
-// (Prod2DTLRec + Upd2DPert) reads them back instead of transforming the base
+// last stage's column pass advances.  The perturbation-only flow
+// (Prod2DTLRec) reads them back instead of transforming the base
 // again, so one tangent-linear step costs the transforms of a plain step.
 // Past the record's last slot nothing is stored and zeros are read; the host
 // sizes the record so that this never happens.
@@ -451,21 +486,6 @@ template <typename P, typename RP> struct Prod2DTLRec {
   }
 };
 
-// the perturbation half of the tangent-linear update
-template <int STAGE> struct Upd2DPert {
-  Upd2DTL<STAGE> t;
-  __device__ __forceinline__ void operator()(int m, long ik, int, double kx, double ky, cpx<double> (&N)[2]) const {
-    t.pert(m, ik, kx, ky, N);
-  }
-};
-
-// the last stage of a recording or replaying step advances the step counter
-template <class U> struct StepEnd : U {
-  static constexpr bool ONCE = true;
-  int *cnt;
-  __device__ __forceinline__ void once() const { *cnt = *cnt + 1; }
-};
-
 __global__ void k2_zero_int(int *p) { *p = 0; }
 
 // the split-row x-pass alone (the record is indexed by row)
@@ -498,24 +518,16 @@ template <typename P, typename RP> static int run2rec_t(Ctx *c, int nsteps, bool
     set_error("recorded base: one member and an allocated record only");
     return PSG_EINVAL;
   }
-  if (first) {
-    hipLaunchKernelGGL(k2_setz0, dim3((unsigned)((g.nkt + 255) / 256 < 4096 ? (g.nkt + 255) / 256 : 4096)),
-                       dim3(256), 0, c->stream, c->state, c->stage, c->mask, g.nkt, g.nkt);
-    PSG_HIP(hipGetLastError());
-  }
-  const double famp = c->cfg.force == PSG_FORCE_NONE ? 0.0 : c->cfg.ampfor;
   cpx<P> *B = (cpx<P> *)c->bufB, *Cb = (cpx<P> *)c->bufC;
+  if (first) PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, B, 1, load2(c, c->state))));
   for (int nt = 0; nt < nsteps; nt++) {
-#define PSG_REC_STAGE(S, UPD)                                                                                \
-    {                                                                                                        \
-      Upd2D<S> u{c->state, c->stage, c->rh, g.nkt, c->mask, c->cfg.dt, c->cfg.v2, famp, c->cfg.kf, nullptr}; \
-      Prod2DRec<P, RP> pr{(RP *)c->rec, c->rec_cnt, S, c->rec_slots, g.nx, g.ny};                            \
-      PSG_TRY2(launch_yinv2<P>(c, c->stage, B, 1));                                                          \
-      PSG_TRY2((launch_xpass2_split<P, 3, 2>(c, B, Cb, pr)));                                               \
-      PSG_TRY2(launch_yfwd2<P>(c, Cb, UPD, 1));                                                              \
+#define PSG_REC_STAGE(S)                                                           \
+    {                                                                              \
+      Prod2DRec<P, RP> pr{(RP *)c->rec, c->rec_cnt, S, c->rec_slots, g.nx, g.ny};  \
+      PSG_TRY2((launch_xpass2_split<P, 3, 2>(c, B, Cb, pr)));                      \
+      PSG_TRY2((launch_col2<P, true, true>(c, Cb, B, 1, upd2<S>(c, c->rec_cnt)))); \
     }
-    PSG_REC_STAGE(0, u) PSG_REC_STAGE(1, u) PSG_REC_STAGE(2, u)
-    PSG_REC_STAGE(3, (StepEnd<Upd2D<3>>{u, c->rec_cnt}))
+    PSG_REC_STAGE(0) PSG_REC_STAGE(1) PSG_REC_STAGE(2) PSG_REC_STAGE(3)
 #undef PSG_REC_STAGE
   }
   return 0;
@@ -527,24 +539,16 @@ template <typename P> static int run2tlrec_t(Ctx *c, int nsteps, bool first) {
     set_error("recorded tangent linear: one member and a record of the pass precision only");
     return PSG_EINVAL;
   }
-  if (first) {
-    hipLaunchKernelGGL(k2_setz0, dim3((unsigned)((g.nkt + 255) / 256 < 4096 ? (g.nkt + 255) / 256 : 4096)),
-                       dim3(256), 0, c->stream, c->tl_state, c->tl_stage, c->mask, g.nkt, g.nkt);
-    PSG_HIP(hipGetLastError());
-  }
   cpx<P> *B = (cpx<P> *)c->tl_bufB, *Cb = (cpx<P> *)c->tl_bufC;
+  if (first) PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, B, 1, load2(c, c->tl_state))));
   for (int nt = 0; nt < nsteps; nt++) {
-#define PSG_TLR_STAGE(S, UPD)                                                                                  \
-    {                                                                                                          \
-      Upd2DPert<S> u{{{c->state, c->stage, c->rh, g.nkt, c->mask, c->cfg.dt, c->cfg.v2, 0.0, c->cfg.kf, nullptr}, \
-                      c->tl_state, c->tl_stage, c->tl_rh}};                                                    \
-      Prod2DTLRec<P, P> pr{(const P *)c->rec, c->rec_cnt, S, c->rec_slots, g.nx, g.ny};                       \
-      PSG_TRY2(launch_yinv2<P>(c, c->tl_stage, B, 1));                                                         \
-      PSG_TRY2((launch_xpass2_split<P, 3, 2>(c, B, Cb, pr)));                                                 \
-      PSG_TRY2(launch_yfwd2<P>(c, Cb, UPD, 1));                                                                \
+#define PSG_TLR_STAGE(S)                                                                \
+    {                                                                                   \
+      Prod2DTLRec<P, P> pr{(const P *)c->rec, c->rec_cnt, S, c->rec_slots, g.nx, g.ny}; \
+      PSG_TRY2((launch_xpass2_split<P, 3, 2>(c, B, Cb, pr)));                           \
+      PSG_TRY2((launch_col2<P, true, true>(c, Cb, B, 1, pert2<S>(c, c->rec_cnt))));     \
     }
-    PSG_TLR_STAGE(0, u) PSG_TLR_STAGE(1, u) PSG_TLR_STAGE(2, u)
-    PSG_TLR_STAGE(3, (StepEnd<Upd2DPert<3>>{u, c->rec_cnt}))
+    PSG_TLR_STAGE(0) PSG_TLR_STAGE(1) PSG_TLR_STAGE(2) PSG_TLR_STAGE(3)
 #undef PSG_TLR_STAGE
   }
   return 0;
@@ -575,10 +579,8 @@ int ns2d_init(Ctx *c) {
   c->szC = (size_t)2 * g.ysz * c->batch * b;
   PSG_HIP(hipMalloc(&c->bufB, c->szB));
   PSG_HIP(hipMalloc(&c->bufC, c->szC));
-  PSG_HIP(hipMalloc(&c->rh, sizeof(cpx<double>) * 3 * g.nkt * c->batch));
-  PSG_HIP(hipMalloc(&c->stage, sizeof(cpx<double>) * g.nkt * c->batch));
-  PSG_HIP(hipMemsetAsync(c->rh, 0, sizeof(cpx<double>) * 3 * g.nkt * c->batch, c->stream));
-  PSG_HIP(hipMemsetAsync(c->stage, 0, sizeof(cpx<double>) * g.nkt * c->batch, c->stream));
+  PSG_HIP(hipMalloc(&c->rh, sizeof(cpx<double>) * g.nkt * c->batch));
+  PSG_HIP(hipMemsetAsync(c->rh, 0, sizeof(cpx<double>) * g.nkt * c->batch, c->stream));
   return 0;
 }
 

@@ -11,8 +11,9 @@
 //   4 yfwd : forward y-FFT, truncation in y      C -> A' [m][FO][NZ][IKTY][XP]
 //   5 zfwd : forward z-FFT, truncation in z, x 1/NR (FP64), then the scheme's
 //            update functor at every stored mode (curl, forcing, mask, CN).
-// 2D uses passes 2-5 shape-wise: y-inverse straight from the state, the same
-// x-pass, and a y-forward pass that ends in the update functor.
+// 2D runs two passes per right-hand side: the x-pass, and a column pass that
+// transforms forward in y, updates the state and transforms the next stage's
+// fields back (k2_col in psg_ns2d.hip).
 //
 // Column passes use a tile of T consecutive kx columns per block (coalesced
 // along the contiguous kx axis) and N/8 threads per column; the x-pass uses
@@ -183,14 +184,26 @@ template <typename P> __device__ __forceinline__ long yoff(const Grid &g, int ik
   constexpr int W = Lay<P>::W, SH = Lay<P>::SH;
   return ((long)z * (g.xp / W) + (ikx >> SH)) * ((long)g.ny * W) + y * W + (ikx & (W - 1));
 }
-// x row rr = z*ny + y of a Y buffer: element k sits at yrow(rr)[ycol(k)]
-template <typename P> __device__ __forceinline__ long yrow(const Grid &g, long rr) {
-  return yoff<P>(g, 0, (int)(rr % g.ny), (int)(rr / g.ny));
-}
-template <typename P> __device__ __forceinline__ int ycol(const Grid &g, int k) {
-  constexpr int W = Lay<P>::W, SH = Lay<P>::SH;
-  return (k >> SH) * (g.ny * W) + (k & (W - 1));
-}
+// x row (y, z) of a Y buffer: element k sits at row(y, z)[col(k)]
+//  YTile: the tiled layout above
+//  YCol : 2D, one kx column after the other ([ikx][y]), for the products too: a
+//         2D column pass owns single columns and reads and writes each as one
+//         run; the x-pass gathers its row from lines that it shares with the
+//         seven rows beside it, which xcd_tile puts on the same XCD
+template <typename P> struct YTile {
+  static __device__ __forceinline__ long row(const Grid &g, int y, int z) { return yoff<P>(g, 0, y, z); }
+  static __device__ __forceinline__ int col(const Grid &g, int k) {
+    constexpr int W = Lay<P>::W, SH = Lay<P>::SH;
+    return (k >> SH) * (g.ny * W) + (k & (W - 1));
+  }
+};
+//         (pitch: columns start an odd number of 128-byte lines apart, so that
+//         the elements of a row spread over the L2 channels)
+struct YCol {
+  static __host__ __device__ __forceinline__ int pitch(const Grid &g) { return g.ny + 8; }
+  static __device__ __forceinline__ long row(const Grid &, int y, int) { return y; }
+  static __device__ __forceinline__ int col(const Grid &g, int k) { return k * pitch(g); }
+};
 
 // Biot-Savart u = i k x w / max(|k|^2,1e-3): 3D_NavierStokes/src/kernels.h:187-201
 __device__ __forceinline__ void biot_savart(double kx, double ky, double kz, cpx<double> xi, cpx<double> et,
@@ -497,9 +510,9 @@ k_zfwd(const cpx<P> *__restrict__ in, Grid g, const cpx<P> *__restrict__ tw, UPD
 // (IKTX = NX/3 + 1 for every grid the context builds)
 template <int N> constexpr int xband() { return N / 3 + 1; }
 
-template <typename P, int N, int E> struct XRow {
+template <typename P, int N, int E, class YL = YTile<P>> struct XRow {
   // pair p of a row: z = a + i b from the half spectra of fields fa, fb, whose
-  // row starts ra, rb hold element k at ycol<P>(g, k)
+  // row starts ra, rb hold element k at YL::col(g, k)
   __device__ __forceinline__ static void load(cpx<P> (&v)[E], const cpx<P> *ra, const cpx<P> *rb, bool hasb,
                                               bool valid, int j, const Grid &g) {
     constexpr int TPX = N / E;
@@ -511,13 +524,13 @@ template <typename P, int N, int E> struct XRow {
       cpx<P> z{0, 0};
       if (valid) {
         if (k < ix) {
-          a = ld_pass<NT<P, PASS_XPASS>::ld>(&ra[ycol<P>(g, k)]);
-          if (hasb) b = ld_pass<NT<P, PASS_XPASS>::ld>(&rb[ycol<P>(g, k)]);
+          a = ld_pass<NT<P, PASS_XPASS>::ld>(&ra[YL::col(g, k)]);
+          if (hasb) b = ld_pass<NT<P, PASS_XPASS>::ld>(&rb[YL::col(g, k)]);
           if (k == 0) { a.y = 0; b.y = 0; }
           z = cpx<P>{a.x - b.y, a.y + b.x};
         } else if (k > N - ix) {
-          a = ld_pass<NT<P, PASS_XPASS>::ld>(&ra[ycol<P>(g, N - k)]);
-          if (hasb) b = ld_pass<NT<P, PASS_XPASS>::ld>(&rb[ycol<P>(g, N - k)]);
+          a = ld_pass<NT<P, PASS_XPASS>::ld>(&ra[YL::col(g, N - k)]);
+          if (hasb) b = ld_pass<NT<P, PASS_XPASS>::ld>(&rb[YL::col(g, N - k)]);
           z = cpx<P>{a.x + b.y, b.x - a.y};
         }
       }
@@ -526,12 +539,20 @@ template <typename P, int N, int E> struct XRow {
   }
 };
 
+// half spectra of the two real fields packed as a + i b, from modes k and -k
+template <typename P>
+__device__ __forceinline__ void split_pair(cpx<P> zk, cpx<P> zc, cpx<P> &A, cpx<P> &B) {
+  const P h = (P)0.5;
+  A = cpx<P>{h * (zk.x + zc.x), h * (zk.y - zc.y)};
+  B = cpx<P>{h * (zk.y + zc.y), h * (zc.x - zk.x)};
+}
+
 // LAZY: the product is re-evaluated per output pair instead of being kept
 // for all outputs, which frees 2*FO*E registers for occupancy.
 // WPE > 0 asks the compiler for at least WPE waves per SIMD (a register cap
 // of 512/WPE VGPRs), trading spills or rematerialisation for occupancy.
 template <typename P, int N, int TEAMS, int FI, int FO, class PROD, int E = EPT, bool FRONT = true,
-          bool LAZY = false, int WPE = 0>
+          bool LAZY = false, int WPE = 0, class YL = YTile<P>>
 __global__ void __launch_bounds__(TEAMS *(N / E)) PSG_WAVES_PER_EU(WPE > 0 ? WPE : 1)
 k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, long nrows, Grid g,
         const cpx<P> *__restrict__ tw, PROD prod, int zs0) {
@@ -544,7 +565,8 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   // row = (m, z, y) with y fastest over the launch's planes zs0 .. zs0 +
   // nrow_m/ny - 1 of each member: the block's first row is split once per
   // block (uniform), each team steps y from it (launches keep nrows < 2^31)
-  const unsigned row0 = blockIdx.x * (unsigned)TEAMS, nrm = (unsigned)nrow_m, ny = (unsigned)g.ny;
+  const unsigned blk = std::is_same<YL, YCol>::value ? (unsigned)xcd_tile().x : blockIdx.x;
+  const unsigned row0 = blk * (unsigned)TEAMS, nrm = (unsigned)nrow_m, ny = (unsigned)g.ny;
   const unsigned m0 = row0 / nrm, rr0 = row0 - m0 * nrm, z0 = rr0 / ny, nzr = nrm / ny;
   unsigned y = rr0 - z0 * ny + team, z = z0, m = m0;
   while (y >= ny) { y -= ny; z++; }
@@ -556,7 +578,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   cpx<P> *tl = lds + team * row_len<N>();
   constexpr int SW = row_swizzle<E>();
   constexpr int ix = xband<N>();
-  const long ro = yoff<P>(g, 0, (int)y, (int)z);
+  const long ro = YL::row(g, (int)y, (int)z);
   auto rowp = [&](int f) { return in + ((long)m * FI + f) * g.ysz + ro; };
   // nine front-loaded fields leave no registers for the twiddles' trip (the
   // FP32 256-point Boussinesq pass ran 0.5% slower with it)
@@ -566,7 +588,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   if constexpr (FRONT) {
 #pragma unroll
     for (int p = 0; p < PI; p++)
-      XRow<P, N, E>::load(vin[p], rowp(2 * p), rowp(2 * p + 1 < FI ? 2 * p + 1 : 2 * p), 2 * p + 1 < FI, valid, j,
+      XRow<P, N, E, YL>::load(vin[p], rowp(2 * p), rowp(2 * p + 1 < FI ? 2 * p + 1 : 2 * p), 2 * p + 1 < FI, valid, j,
                           g);
   }
   if constexpr (!TWFIRST) PSG_TWIDDLES_READY(P);
@@ -579,7 +601,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
 #pragma unroll
       for (int mm = 0; mm < E; mm++) v[mm] = vin[p][mm];
     } else {
-      XRow<P, N, E>::load(v, rowp(fa), rowp(fb < FI ? fb : fa), fb < FI, valid, j, g);
+      XRow<P, N, E, YL>::load(v, rowp(fa), rowp(fb < FI ? fb : fa), fb < FI, valid, j, g);
     }
     fft_pencil<P, N, E, true, WAVE, SW>(v, tl, j, 1, 0, tw);
 #pragma unroll
@@ -625,17 +647,35 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
       const int k = j + TPX * mm;   // only the kept modes and their mirrors are read back
       if (k < ix || k > N - ix) tl[lpos<SW>(k)] = v[mm];
     }
-    team_sync<WAVE>();
-    if (valid) {
-      cpx<P> *oa = out + ((long)m * FO + 2 * q) * g.ysz + rr * g.xp;
-      cpx<P> *ob = out + ((long)m * FO + 2 * q + 1) * g.ysz + rr * g.xp;
-      for (int k = j; k < ix; k += TPX) {
-        cpx<P> zk = tl[lpos<SW>(k)], zc = tl[lpos<SW>((N - k) & (N - 1))];
-        const P h = (P)0.5;
-        cpx<P> A{h * (zk.x + zc.x), h * (zk.y - zc.y)};
-        cpx<P> B{h * (zk.y + zc.y), h * (zc.x - zk.x)};
-        st_pass<NT<P, PASS_XPASS>::st>(&oa[k], A);
-        if (2 * q + 1 < FO) st_pass<NT<P, PASS_XPASS>::st>(&ob[k], B);
+    if constexpr (std::is_same<YL, YCol>::value) {
+      // columns of C: the block's rows lie next to each other in a column, so
+      // its threads take (kx, row) with the row fastest
+      __syncthreads();
+      constexpr int NTH = TEAMS * TPX;
+      for (int i = threadIdx.x; i < ix * TEAMS; i += NTH) {
+        const int r = i % TEAMS, k = i / TEAMS;
+        const unsigned rw = row0 + r, mr = rw / nrm;
+        if (rw < (unsigned long)nrows) {
+          const cpx<P> *tr = lds + r * row_len<N>();
+          cpx<P> A, B;
+          split_pair(tr[lpos<SW>(k)], tr[lpos<SW>((N - k) & (N - 1))], A, B);
+          cpx<P> *o = out + ((long)mr * FO + 2 * q) * g.ysz + YL::col(g, k) + (rw - mr * nrm);
+          o[0] = A;
+          if (2 * q + 1 < FO) o[g.ysz] = B;
+        }
+      }
+      __syncthreads();
+    } else {
+      team_sync<WAVE>();
+      if (valid) {
+        cpx<P> *oa = out + ((long)m * FO + 2 * q) * g.ysz + rr * g.xp;
+        cpx<P> *ob = oa + g.ysz;
+        for (int k = j; k < ix; k += TPX) {
+          cpx<P> A, B;
+          split_pair(tl[lpos<SW>(k)], tl[lpos<SW>((N - k) & (N - 1))], A, B);
+          st_pass<NT<P, PASS_XPASS>::st>(&oa[k], A);
+          if (2 * q + 1 < FO) st_pass<NT<P, PASS_XPASS>::st>(&ob[k], B);
+        }
       }
     }
   }
@@ -654,10 +694,6 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
 // bind(member, row, team) returning an object called as (n, in, out).
 template <class T, class = void> struct prod_row : std::false_type {};
 template <class T> struct prod_row<T, std::void_t<decltype(T::ROW)>> : std::bool_constant<T::ROW> {};
-// An update that must act once per launch (the step counter of the recorded
-// base) provides once(), called by one thread of the first tile.
-template <class T, class = void> struct upd_once : std::false_type {};
-template <class T> struct upd_once<T, std::void_t<decltype(T::ONCE)>> : std::bool_constant<T::ONCE> {};
 
 template <int FI, int FO> constexpr int xsplit_teams() { return (FI + 1) / 2 > (FO + 1) / 2 ? (FI + 1) / 2 : (FO + 1) / 2; }
 template <typename P, int N, int FI, int FO>
@@ -678,17 +714,17 @@ k_xpass_split(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow
   constexpr int SW = row_swizzle<E>();
   constexpr int ix = xband<N>();
   const int team = threadIdx.x / TPX, j = threadIdx.x % TPX;
-  const unsigned row = blockIdx.x, nrm = (unsigned)nrow_m, ny = (unsigned)g.ny;
+  const unsigned row = (unsigned)xcd_tile().x, nrm = (unsigned)nrow_m, ny = (unsigned)g.ny;
   const bool valid = row < (unsigned long)nrows;
   const unsigned m = valid ? row / nrm : 0, rr = valid ? row - m * nrm : 0, z = rr / ny, y = rr - z * ny;
   cpx<P> *tl = lds + team * row_len<N>();
   P *phys = reinterpret_cast<P *>(lds + NTEAM * row_len<N>());
-  const long ro = yoff<P>(g, 0, (int)y, (int)z);
+  const long ro = YCol::row(g, (int)y, (int)z);
   auto rowp = [&](int f) { return in + ((long)m * FI + f) * g.ysz + ro; };
   {
     const int p = team < PI ? team : PI - 1, fa = 2 * p, fb = 2 * p + 1;
     cpx<P> v[E];
-    XRow<P, N, E>::load(v, rowp(fa), rowp(fb < FI ? fb : fa), fb < FI, valid && team < PI, j, g);
+    XRow<P, N, E, YCol>::load(v, rowp(fa), rowp(fb < FI ? fb : fa), fb < FI, valid && team < PI, j, g);
     PSG_TWIDDLES_READY(P);
     fft_pencil<P, N, E, true, WAVE, SW>(v, tl, j, 1, 0, tw);
     if (team < PI) {
@@ -729,15 +765,12 @@ k_xpass_split(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow
   }
   team_sync<WAVE>();
   if (valid && team < PO) {
-    cpx<P> *oa = out + ((long)m * FO + 2 * q) * g.ysz + (long)rr * g.xp;
-    cpx<P> *ob = out + ((long)m * FO + 2 * q + 1) * g.ysz + (long)rr * g.xp;
+    cpx<P> *oa = out + ((long)m * FO + 2 * q) * g.ysz + YCol::row(g, (int)y, 0);
     for (int k = j; k < ix; k += TPX) {
-      cpx<P> zk = tl[lpos<SW>(k)], zc = tl[lpos<SW>((N - k) & (N - 1))];
-      const P h = (P)0.5;
-      cpx<P> A{h * (zk.x + zc.x), h * (zk.y - zc.y)};
-      cpx<P> B{h * (zk.y + zc.y), h * (zc.x - zk.x)};
-      st_pass<false>(&oa[k], A);   // 2D grids: the y-forward reads C back from the caches
-      if (2 * q + 1 < FO) st_pass<false>(&ob[k], B);
+      cpx<P> A, B;
+      split_pair(tl[lpos<SW>(k)], tl[lpos<SW>((N - k) & (N - 1))], A, B);
+      oa[YCol::col(g, k)] = A;
+      if (2 * q + 1 < FO) oa[g.ysz + YCol::col(g, k)] = B;
     }
   }
 }
@@ -773,120 +806,5 @@ template <typename P> struct Prod2D {
     out[1] = in[1] * in[0];
   }
 };
-
-// ---------------------------------------------------------------- 2D passes
-// y-inverse straight from the state: Hermitian fill of kx=0 (in place in the
-// reference, 2D_NavierStokes/src_RK4/kernels.h:82-96), mask, Biot-Savart
-// (kernels.h:112-147), zero-pad, inverse y-FFT.  out fields w,u,v.
-// SPLIT: blockIdx.y picks one of the 3*NSRC output fields (3*NSRC times the
-// blocks, for grids too small to fill the GPU with column tiles alone)
-template <typename P, int N, int T, int NSRC = 1, bool SPLIT = false>
-__global__ void __launch_bounds__(T *(N / EPT))
-k2_yinv(const cpx<double> *__restrict__ st, long st_ms, cpx<P> *__restrict__ out, long out_ms, Grid g,
-        const cpx<P> *__restrict__ tw, const int8_t *__restrict__ mask,
-        const cpx<double> *__restrict__ st2 = nullptr) {
-  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
-  PSG_TWIDDLES_READY(P);
-  constexpr int TP = N / EPT;
-  const int col = threadIdx.x % T, j = threadIdx.x / T;
-  const TileId tid = xcd_tile();
-  const int ikx = tid.x * T + col, m = tid.z, sel = tid.y;
-  const bool valid = ikx < g.iktx;
-  const double kx = (double)ikx * g.alpha;
-#pragma unroll 1
-  for (int src = 0; src < NSRC; src++) {
-    if (SPLIT && src != sel / 3) continue;
-    const cpx<double> *s0 = (src == 0 ? st : st2) + (long)m * st_ms;
-    cpx<double> w[EPT];
-    double kyv[EPT];
-#pragma unroll
-    for (int mm = 0; mm < EPT; mm++) {
-      const int y = j + TP * mm;
-      const int ky = wrapk(y, g.ny, g.kty);
-      cpx<double> a{0, 0};
-      kyv[mm] = ky == PSG_NOK ? 0.0 : (double)ky;
-      if (valid && ky != PSG_NOK) {
-        if (ikx == 0 && ky < 0) {
-          long idx = (long)(-ky + g.kty) * g.iktx;
-          if (mask[idx]) { a = s0[idx]; a.y = -a.y; }
-        } else {
-          long idx = (long)(ky + g.kty) * g.iktx + ikx;
-          if (mask[idx]) a = s0[idx];
-        }
-      }
-      w[mm] = a;
-    }
-#pragma unroll
-    for (int f = 0; f < 3; f++) {
-      if (SPLIT && f != sel % 3) continue;
-      cpx<P> v[EPT];
-#pragma unroll
-      for (int mm = 0; mm < EPT; mm++) {
-        if (f == 0) v[mm] = to<P>(w[mm]);
-        else {
-          const double ky = kyv[mm];
-          const double wk = kx * kx + ky * ky;
-          const double wki = 1.0 / (wk > 0.001 ? wk : 0.001);
-          cpx<double> r;
-          if (f == 1) r = cpx<double>{-ky * w[mm].y * wki, ky * w[mm].x * wki};
-          else r = cpx<double>{kx * w[mm].y * wki, -kx * w[mm].x * wki};
-          v[mm] = to<P>(r);
-        }
-      }
-      fft_pencil<P, N, EPT, true>(v, lds, j, T, col, tw);
-      if (valid) {
-        cpx<P> *o = out + (long)m * out_ms + (long)(3 * src + f) * g.ysz;
-#pragma unroll
-        for (int mm = 0; mm < EPT; mm++) st_pass<false>(&o[yoff<P>(g, ikx, j + TP * mm, 0)], v[mm]);   // 2D: the next pass reads it from cache
-      }
-    }
-  }
-}
-
-// y-forward + update (2D).  UPD::operator()(m, ik, ikx, kx, ky, N[2]) with
-// N[0] = FFT(v w)/NR, N[1] = FFT(u w)/NR  (the reference's NZK halves).
-// NG > 1: the NF fields form NG independent groups, blockIdx.y picks one and
-// its update is UPD::part(group, m, ik, ikx, kx, ky, N[NF/NG]).
-template <typename P, int N, int T, class UPD, int NF = 2, int NG = 1>
-__global__ void __launch_bounds__(T *(N / EPT))
-k2_yfwd(const cpx<P> *__restrict__ in, long in_ms, Grid g, const cpx<P> *__restrict__ tw, UPD upd) {
-  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
-  PSG_TWIDDLES_READY(P);
-  constexpr int TP = N / EPT, NFG = NF / NG;
-  const int col = threadIdx.x % T, j = threadIdx.x / T;
-  const TileId tid = xcd_tile();
-  const int ikx = tid.x * T + col, m = tid.z, grp = NG > 1 ? tid.y : 0;
-  const bool valid = ikx < g.iktx;
-  cpx<double> res[NFG][EPT];
-#pragma unroll
-  for (int f = 0; f < NFG; f++) {
-    const cpx<P> *src = in + (long)m * in_ms + (long)(grp * NFG + f) * g.ysz + ikx;
-    cpx<P> v[EPT];
-#pragma unroll
-    for (int mm = 0; mm < EPT; mm++) v[mm] = valid ? src[(long)(j + TP * mm) * g.xp] : cpx<P>{0, 0};
-    fft_pencil<P, N, EPT, false>(v, lds, j, T, col, tw);
-#pragma unroll
-    for (int mm = 0; mm < EPT; mm++) {
-      cpx<double> t = up(v[mm]);
-      res[f][mm] = cpx<double>{t.x * g.inr, t.y * g.inr};
-    }
-  }
-  if constexpr (upd_once<UPD>::value) {
-    if (tid.x == 0 && tid.y == 0 && tid.z == 0 && threadIdx.x == 0) upd.once();
-  }
-  if (!valid) return;
-  const double kx = (double)ikx * g.alpha;
-#pragma unroll
-  for (int mm = 0; mm < EPT; mm++) {
-    const int ky = wrapk(j + TP * mm, g.ny, g.kty);
-    if (ky == PSG_NOK) continue;
-    const long ik = (long)(ky + g.kty) * g.iktx + ikx;
-    cpx<double> nn[NFG];
-#pragma unroll
-    for (int f = 0; f < NFG; f++) nn[f] = res[f][mm];
-    if constexpr (NG > 1) upd.part(grp, m, ik, ikx, kx, (double)ky, nn);
-    else upd(m, ik, ikx, kx, (double)ky, nn);
-  }
-}
 
 }  // namespace psg
