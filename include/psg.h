@@ -165,6 +165,10 @@ int psg_device_count(void);
  *   v  the three passes over 128 >> (v-1) planes at a time (128, 64, 32, 16, 8),
  *      so that a slab's intermediate buffers are read back from the device's
  *      last-level cache instead of HBM
+ * Variant 0 of all three passes is the context's default stepper: on small grids
+ * (32 to 128 points an extent, buffers within a quarter of the last-level cache)
+ * that is a two-kernel form of the right-hand side, and the shapes above, of the
+ * five pencil passes, are taken by any other choice.
  * psg_autotune times `steps` steps of every variant of each pass in turn on the
  * context's own state (restored afterwards), keeps the fastest of each and
  * writes a text report. */

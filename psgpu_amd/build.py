@@ -32,7 +32,7 @@ HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-Wall", "-
 C_FLAGS = ["-O2", "-fPIC", "-std=gnu11", "-Wall", "-I" + os.path.join(ROOT, "include")]
 
 CORE_HIP = ["psg_api.hip", "psg_ns3d.hip", "psg_ns2d.hip", "psg_bous.hip", "psg_newton.hip", "psg_tladj.hip",
-            "psg_rec.hip", "psg_stats.hip"]
+            "psg_rec.hip", "psg_stats.hip", "psg_split64.hip", "psg_split32.hip"]
 CORE_C = ["psg_host.c"]
 CXX20_HIP = {"psg_newton.hip"}   # the Newton solver is a C++20 coroutine
 # legacy shims: (library suffix, source)

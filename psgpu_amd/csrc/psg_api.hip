@@ -616,6 +616,8 @@ int psg_create(const psg_config *cfg, psg_ctx **out) {
   g.inr = 1.0 / (double)hg.nr;
   g.kmax2 = ((double)g.kty - 0.5) * ((double)g.kty - 0.5);
   hipGetDevice(&c->device);
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0) c->cus = cus;
   int rc = 0;
   do {
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { rc = PSG_EHIP; set_error("stream"); break; }

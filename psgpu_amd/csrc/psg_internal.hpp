@@ -50,18 +50,21 @@ struct Ctx {
   int batch;
   hipStream_t stream = nullptr;
   int device = 0;
+  int cus = 256;   // compute units of the device
   // state and scheme arrays (FP64 complex), member-major [batch][nf][nkt]
   cpx<double> *state = nullptr;
   cpx<double> *rh = nullptr;        // Heun: RH store; RK4: stage arrays
   cpx<double> *stage = nullptr;     // RK4: Z0 stage input / generic scratch
   cpx<double> *tmp = nullptr;       // scratch state-sized buffer
   // 3D Navier-Stokes/Euler: working copy of the state during a run, in the
-  // z-run layout LayW (FP64, or FP32 in FP32-bulk), and the CN tables and
-  // mask in the same order (nktw modes per field, IKTX rounded up to 8)
+  // layout LayW of the five pencil passes or Split::at of the two-kernel
+  // stepper (FP64, or FP32 in FP32-bulk), and the CN tables and mask in the
+  // same order (nktw modes per field in LayW, IKTX rounded up to 8)
   cpx<double> *stw = nullptr;
   cpx<float> *st32 = nullptr;
   bool work_live = false;           // the working copy holds the current state (inside run_steps)
   long nktw = 0;
+  bool wsplit = false;              // layout of the working copy and its tables: LayW, or Split::at
   double *wnuzn = nullptr, *wnu1 = nullptr;
   int8_t *wmask = nullptr;
   double *nuzn = nullptr, *nu1 = nullptr;  // CN tables (host-built, reference formula)

@@ -12,6 +12,7 @@
 // is the same Biot-Savart expression and saves 6 NKT complex of traffic.
 #include <type_traits>
 #include "psg_ns3d.hpp"
+#include "psg_split.hpp"
 
 namespace psg {
 
@@ -263,6 +264,46 @@ template <typename A, typename B, bool TO_W> static int work_copy(Ctx *c, const 
   return 0;
 }
 
+// The same for the two-kernel stepper's layout (Split::at), whose runs go along
+// kz: 16 kx x 64 kz tiles turn through LDS so that both sides move whole runs.
+// One (iky, member, field) per blockIdx.y, z.
+constexpr int WTX = 16, WTZ = 64;
+template <typename A, typename B, bool TO_W>
+__global__ void __launch_bounds__(256) k_work_split(const cpx<A> *__restrict__ a, cpx<B> *__restrict__ b, Grid g, Split d) {
+  PSG_DYN_SMEM(smem_raw);
+  cpx<B> *t = reinterpret_cast<cpx<B> *>(smem_raw);
+  const int ntx = (g.iktx + WTX - 1) / WTX, x0 = (int)(blockIdx.x % ntx) * WTX, z0 = (int)(blockIdx.x / ntx) * WTZ;
+  const int iky = blockIdx.y, m = blockIdx.z / 3, f = blockIdx.z % 3;
+  const long an = (long)blockIdx.z * g.nkt, wn = (long)m * 3 * d.nkts + (long)f * d.kzp;
+  for (int h = 0; h < 2; h++) {
+    const bool kxfast = (h == 0) == TO_W;   // the reference order's side
+    for (int i = threadIdx.x; i < WTX * WTZ; i += 256) {
+      const int lx = kxfast ? i % WTX : i / WTZ, lz = kxfast ? i / WTX : i % WTZ;
+      const int ikx = x0 + lx, c = z0 + lz;   // c: kz in the working order
+      if (ikx >= g.iktx || c >= g.iktz) continue;
+      const int ikz = c <= g.ktz ? c + g.ktz : c - g.ktz - 1;
+      const long n = an + LayNKT::at(g, ikx, iky, ikz), w = wn + ((long)ikx * g.ikty + iky) * 3 * d.kzp + c;
+      cpx<B> &slot = t[lx * (WTZ + 1) + lz];
+      if (h == 0) {
+        const cpx<A> v = a[TO_W ? n : w];
+        slot = cpx<B>{(B)v.x, (B)v.y};
+      } else {
+        b[TO_W ? w : n] = slot;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+template <typename A, typename B, bool TO_W> static int work_copy_split(Ctx *c, const cpx<A> *a, cpx<B> *b) {
+  const Grid &g = c->g;
+  const unsigned nt = (unsigned)(((g.iktx + WTX - 1) / WTX) * ((g.iktz + WTZ - 1) / WTZ));
+  hipLaunchKernelGGL((k_work_split<A, B, TO_W>), dim3(nt, g.ikty, 3 * c->batch), dim3(256),
+                     sizeof(cpx<B>) * WTX * (WTZ + 1), c->stream, a, b, g, Split::of(g));
+  PSG_HIP(hipGetLastError());
+  return 0;
+}
+
 // CN tables and mask in the working layout (zero at padding columns)
 __global__ void k_tables_w(const double *__restrict__ nuzn, const double *__restrict__ nu1,
                            const int8_t *__restrict__ L, double *__restrict__ wnuzn, double *__restrict__ wnu1,
@@ -281,8 +322,31 @@ __global__ void k_tables_w(const double *__restrict__ nuzn, const double *__rest
   }
 }
 
+// in Split::at's order (padding along kz is never read)
+__global__ void k_tables_split(const double *__restrict__ nuzn, const double *__restrict__ nu1,
+                               const int8_t *__restrict__ L, double *__restrict__ wnuzn, double *__restrict__ wnu1,
+                               int8_t *__restrict__ wL, Grid g, Split d) {
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < d.nkts; i += (long)gridDim.x * blockDim.x) {
+    const int c = (int)(i % d.kzp);
+    const long t = i / d.kzp;
+    const int iky = (int)(t % g.ikty), ikx = (int)(t / g.ikty), ikz = c <= g.ktz ? c + g.ktz : c - g.ktz - 1;
+    const bool in = c < g.iktz;
+    const long n = LayNKT::at(g, ikx, iky, in ? ikz : 0);
+    wnuzn[i] = in ? nuzn[n] : 0.0;
+    wnu1[i] = in ? nu1[n] : 0.0;
+    wL[i] = in ? L[n] : (int8_t)0;
+  }
+}
+
 int ns3d_tables_w(Ctx *c) {
   if (!c->wnuzn) return 0;
+  if (c->wsplit) {
+    const Split d = Split::of(c->g);
+    hipLaunchKernelGGL(k_tables_split, dim3((unsigned)std::min<long>(4096, (d.nkts + 255) / 256)), dim3(256), 0, c->stream,
+                       c->nuzn, c->nu1, c->mask, c->wnuzn, c->wnu1, c->wmask, c->g, d);
+    PSG_HIP(hipGetLastError());
+    return 0;
+  }
   hipLaunchKernelGGL(k_tables_w, dim3((unsigned)std::min<long>(4096, (c->nktw + 255) / 256)), dim3(256), 0, c->stream,
                      c->nuzn, c->nu1, c->mask, c->wnuzn, c->wnu1, c->wmask, c->g, c->nktw);
   PSG_HIP(hipGetLastError());
@@ -298,7 +362,14 @@ int ns3d_tables_w(Ctx *c) {
 // this way).
 int ns3d_work_begin(Ctx *c) {
   if (c->work_live) return 0;
-  if (c->st32) PSG_TRY((work_copy<double, float, true>(c, c->state, c->st32)));
+  if (split_usable(c) != c->wsplit) {
+    c->wsplit = !c->wsplit;
+    PSG_TRY(ns3d_tables_w(c));
+  }
+  if (c->wsplit) {
+    if (c->st32) PSG_TRY((work_copy_split<double, float, true>(c, c->state, c->st32)));
+    else PSG_TRY((work_copy_split<double, double, true>(c, c->state, c->stw)));
+  } else if (c->st32) PSG_TRY((work_copy<double, float, true>(c, c->state, c->st32)));
   else PSG_TRY((work_copy<double, double, true>(c, c->state, c->stw)));
   c->work_live = true;
   return 0;
@@ -307,6 +378,9 @@ int ns3d_work_begin(Ctx *c) {
 int ns3d_work_end(Ctx *c) {
   if (!c->work_live) return 0;
   c->work_live = false;
+  if (c->wsplit)
+    return c->st32 ? work_copy_split<float, double, false>(c, c->st32, c->state)
+                   : work_copy_split<double, double, false>(c, c->stw, c->state);
   if (c->st32) return work_copy<float, double, false>(c, c->st32, c->state);
   return work_copy<double, double, false>(c, c->stw, c->state);
 }
@@ -314,7 +388,9 @@ int ns3d_work_end(Ctx *c) {
 int ns3d_run(Ctx *c, int nsteps, bool first) {
   const bool own = !c->work_live;
   if (own) PSG_TRY(ns3d_work_begin(c));
-  const int r = c->st32 ? run_t<float, float>(c, c->st32, nsteps, first) : run_t<double, double>(c, c->stw, nsteps, first);
+  const int r = c->wsplit ? (c->st32 ? split_run<float>(c, c->st32, nsteps, first) : split_run<double>(c, c->stw, nsteps, first))
+                          : (c->st32 ? run_t<float, float>(c, c->st32, nsteps, first)
+                                     : run_t<double, double>(c, c->stw, nsteps, first));
   if (!own) return r;
   const int r2 = ns3d_work_end(c);
   return r ? r : r2;
@@ -427,20 +503,29 @@ int ns3d_init(Ctx *c) {
   c->szA = (size_t)6 * g.zsz * c->batch * b;
   c->szB = (size_t)6 * g.ysz * c->batch * b;
   c->szC = (size_t)3 * g.ysz * c->batch * b;
+  // the two-kernel stepper keeps F in bufB and G in bufC
+  c->wsplit = split_usable(c);
+  const Split d = Split::of(g);
+  if (c->wsplit) {
+    c->szB = std::max(c->szB, (size_t)6 * d.fs * c->batch * b);
+    c->szC = std::max(c->szC, (size_t)3 * d.gs * c->batch * b);
+  }
   PSG_HIP(hipMalloc(&c->bufA, c->szA));
   PSG_HIP(hipMalloc(&c->bufB, c->szB));
   PSG_HIP(hipMalloc(&c->bufC, c->szC));
-  // RH serves the working-layout stepper and the reference-order steps of
-  // the adjoint's recorded trajectory: the larger of the two sizes
+  // RH serves the steppers in both working layouts and the reference-order
+  // steps of the adjoint's recorded trajectory: the largest of the sizes
   c->nktw = (long)((g.iktx + 7) / 8) * 8 * g.ikty * g.iktz;
-  const long nrh = 3 * std::max<long>(c->nktw, g.nkt) * c->batch;
+  const long nw = c->wsplit ? std::max(c->nktw, d.nkts) : c->nktw;
+  const long ncopy = c->wsplit ? std::max(c->nktw, 2 * d.nkts) : c->nktw;   // the two-kernel stepper keeps two copies
+  const long nrh = 3 * std::max<long>(nw, g.nkt) * c->batch;
   PSG_HIP(hipMalloc(&c->rh, sizeof(cpx<double>) * nrh));
   PSG_HIP(hipMemsetAsync(c->rh, 0, sizeof(cpx<double>) * nrh, c->stream));
-  if (c->cfg.precision == PSG_FP32BULK) PSG_HIP(hipMalloc(&c->st32, sizeof(cpx<float>) * 3 * c->nktw * c->batch));
-  else PSG_HIP(hipMalloc(&c->stw, sizeof(cpx<double>) * 3 * c->nktw * c->batch));
-  PSG_HIP(hipMalloc(&c->wnuzn, sizeof(double) * c->nktw));
-  PSG_HIP(hipMalloc(&c->wnu1, sizeof(double) * c->nktw));
-  PSG_HIP(hipMalloc(&c->wmask, c->nktw));
+  if (c->cfg.precision == PSG_FP32BULK) PSG_HIP(hipMalloc(&c->st32, sizeof(cpx<float>) * 3 * ncopy * c->batch));
+  else PSG_HIP(hipMalloc(&c->stw, sizeof(cpx<double>) * 3 * ncopy * c->batch));
+  PSG_HIP(hipMalloc(&c->wnuzn, sizeof(double) * nw));
+  PSG_HIP(hipMalloc(&c->wnu1, sizeof(double) * nw));
+  PSG_HIP(hipMalloc(&c->wmask, nw));
   return ns3d_tables_w(c);
 }
 

@@ -608,6 +608,13 @@ int main(int argc, char **argv) {
     snprintf(nm, sizeof nm, "ns3d 32^3 fp32 xpass variant %d", v);
     ns3d_case(nm, PSG_NS3D, 32, 32, 32, 1.0, PSG_FP32BULK, v, 0, 2, PSG_FORCE_KOLMO, 1e-4);
   }
+  // the two-kernel stepper (32 points and more an extent, default shapes)
+  ns3d_case("ns3d 32^3 fp64 two kernels", PSG_NS3D, 32, 32, 32, 1.0, PSG_FP64, 0, 0, 2, PSG_FORCE_KOLMO, 1e-12);
+  ns3d_case("euler 32x64x32 fp64 two kernels batch 2", PSG_EULER3D, 32, 64, 32, 2.0, PSG_FP64, 0, 0, 2, PSG_FORCE_NONE,
+            1e-12, 0, 0, 2);
+  ns3d_case("ns3d 32x32x64 fp32 two kernels batch 2", PSG_NS3D, 32, 32, 64, 1.0, PSG_FP32BULK, 0, 0, 2, PSG_FORCE_DNS, 1e-5,
+            0, 0, 2);
+  ns3d_case("ns3d 64x32x32 fp64 two kernels graph", PSG_NS3D, 64, 32, 32, 0.5, PSG_FP64, 0, 2, 4, PSG_FORCE_GMRES, 1e-12);
   ns3d_case("ns3d 16^3 fp64 zfwd variant 1", PSG_NS3D, 16, 16, 16, 1.0, PSG_FP64, 0, 0, 2, PSG_FORCE_KOLMO, 1e-11, 1);
   // passes 2-4 by slabs of z planes: 16 and 8 planes of 32, batches of 2, graph path
   ns3d_case("ns3d 32^3 fp64 slabs of 16", PSG_NS3D, 32, 32, 32, 1.0, PSG_FP64, 1, 0, 2, PSG_FORCE_KOLMO, 1e-11, 0, 4);

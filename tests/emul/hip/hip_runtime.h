@@ -30,6 +30,7 @@
 #define __forceinline__ inline
 #define __launch_bounds__(...)
 #define PSG_WAVES_PER_EU(...)
+#define PSG_FRESH(i) ((void)0)
 #define __shared__ static thread_local
 #define PSG_DYN_SMEM(name) char *name = ::emu::dyn_smem
 #define __align__(n) __attribute__((aligned(n)))
@@ -117,6 +118,8 @@ inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
 inline hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
+enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount };
+inline hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 2; return hipSuccess; }
 inline hipError_t hipMalloc(void **p, size_t n) {
   *p = malloc(n ? n : 1);
   return *p ? hipSuccess : hipErrorMemoryAllocation;
