@@ -21,7 +21,7 @@ template <typename P, int N, int T>
 __global__ void __launch_bounds__(T *(N / EPT))
 k_zinv_bous(const cpx<double> *__restrict__ st, long st_ms, long fs, cpx<P> *__restrict__ out, long out_ms, Grid g,
             const cpx<P> *__restrict__ tw, const int8_t *__restrict__ mask, int umask, int nout) {
-  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
+  PSG_TWIDDLES_REQUEST(P, N, EPT, T *(N / EPT));
   PSG_TWIDDLES_READY(P);
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;

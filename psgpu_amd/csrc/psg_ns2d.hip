@@ -142,7 +142,7 @@ k2_col(const cpx<P> *__restrict__ in, long in_ms, cpx<P> *__restrict__ out, long
   constexpr int NI = (2 * (N / 3) + 1 + NT - 1) / NT;   // modes of the column per thread
   constexpr bool WAVE = TP <= 64;
   constexpr int SW = row_swizzle<EPT>();
-  PSG_LDS_TWIDDLES(P, N, EPT, NT);
+  PSG_TWIDDLES_REQUEST(P, N, EPT, NT);
   const int team = threadIdx.x / TP, j = threadIdx.x % TP;
   const TileId tid = xcd_tile();
   const int ikx = tid.x, grp = NG > 1 ? tid.y : 0, m = tid.z;
@@ -331,7 +331,7 @@ int ns2d_nonlin(Ctx *c, int, const cpx<double> *in_dev, cpx<double> *out_dev) {
 template <typename P, int N, int TE>
 __global__ void __launch_bounds__(TE *(N / EPT))
 k2_xphys(const cpx<P> *__restrict__ in, double *__restrict__ out, long nrow, Grid g, const cpx<P> *__restrict__ tw) {
-  PSG_LDS_TWIDDLES(P, N, EPT, TE *(N / EPT));
+  PSG_TWIDDLES_REQUEST(P, N, EPT, TE *(N / EPT));
   constexpr int TPX = N / EPT;
   const int team = threadIdx.x / TPX, j = threadIdx.x % TPX;
   const long row = (long)blockIdx.x * TE + team;

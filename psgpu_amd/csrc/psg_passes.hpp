@@ -102,7 +102,7 @@ __device__ __forceinline__ TileId xcd_tile() {
 #endif
 // LDS of a transform kernel of NT threads and its share of the twiddles;
 // PSG_TWIDDLES_READY goes after the requests of the block's first data
-#define PSG_LDS_TWIDDLES(P, N, E, NT)                                  \
+#define PSG_TWIDDLES_REQUEST(P, N, E, NT)                                  \
   PSG_DYN_SMEM(smem_raw);                                              \
   cpx<P> *lds = reinterpret_cast<cpx<P> *>(smem_raw) + (N);            \
   Twiddles<P, N, E, (NT)> tws;                                         \
@@ -287,7 +287,7 @@ template <typename P, int N, int T, bool BS, typename S = double, class LAY = La
 __global__ void __launch_bounds__(T *(N / EPT))
 k_zinv(const cpx<S> *__restrict__ st, long st_ms, long st_fs, cpx<P> *__restrict__ out, long out_ms, Grid g,
        const cpx<P> *__restrict__ tw, const int8_t *__restrict__ mask, int umask) {
-  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
+  PSG_TWIDDLES_REQUEST(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -362,7 +362,7 @@ k_zinv(const cpx<S> *__restrict__ st, long st_ms, long st_fs, cpx<P> *__restrict
 template <typename P, int N, int T>
 __global__ void __launch_bounds__(T *(N / EPT))
 k_yinv(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cpx<P> *__restrict__ tw, int z0) {
-  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
+  PSG_TWIDDLES_REQUEST(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -389,7 +389,7 @@ k_yinv(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cp
 template <typename P, int N, int T>
 __global__ void __launch_bounds__(T *(N / EPT))
 k_yfwd(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cpx<P> *__restrict__ tw, int z0) {
-  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
+  PSG_TWIDDLES_REQUEST(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
@@ -423,7 +423,7 @@ template <typename P, int N, int T, int FO, class UPD, bool FRONT = (FO <= 4), i
 __global__ void __launch_bounds__(T *(N / EPT))
 k_zfwd(const cpx<P> *__restrict__ in, Grid g, const cpx<P> *__restrict__ tw, UPD upd) {
   static_assert(PIPE == 1 || FRONT, "row pipelining needs front-loaded inputs");
-  PSG_LDS_TWIDDLES(P, N, EPT, T *(N / EPT));
+  PSG_TWIDDLES_REQUEST(P, N, EPT, T *(N / EPT));
   constexpr int TP = N / EPT;
   constexpr int NV = FRONT ? FO : 1;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
@@ -556,7 +556,7 @@ template <typename P, int N, int TEAMS, int FI, int FO, class PROD, int E = EPT,
 __global__ void __launch_bounds__(TEAMS *(N / E)) PSG_WAVES_PER_EU(WPE > 0 ? WPE : 1)
 k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, long nrows, Grid g,
         const cpx<P> *__restrict__ tw, PROD prod, int zs0) {
-  PSG_LDS_TWIDDLES(P, N, E, TEAMS *(N / E));
+  PSG_TWIDDLES_REQUEST(P, N, E, TEAMS *(N / E));
   constexpr int TPX = N / E;
   constexpr bool WAVE = TPX <= 64;
   constexpr int PI = (FI + 1) / 2, PO = (FO + 1) / 2;
@@ -707,7 +707,7 @@ __global__ void __launch_bounds__((xsplit_teams<FI, FO>() * (N / E)))
 k_xpass_split(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, long nrows, Grid g,
               const cpx<P> *__restrict__ tw, PROD prod) {
   constexpr int NTH = xsplit_teams<FI, FO>() * (N / E);
-  PSG_LDS_TWIDDLES(P, N, E, NTH);
+  PSG_TWIDDLES_REQUEST(P, N, E, NTH);
   constexpr int TPX = N / E;
   constexpr bool WAVE = TPX <= 64;
   constexpr int PI = (FI + 1) / 2, PO = (FO + 1) / 2, NTEAM = xsplit_teams<FI, FO>();

@@ -104,7 +104,7 @@ k_zsplit(const cpx<P> *__restrict__ G, cpx<P> *__restrict__ F, const cpx<P> *__r
   using Z = ZShape<NZ, RA>;
   constexpr int E = EPT, TP = Z::TP, NT = Z::NT, KB = Z::KB, COLS = Z::COLS;
   constexpr int SW = row_swizzle<E>();
-  PSG_LDS_TWIDDLES(P, NZ, E, NT);
+  PSG_TWIDDLES_REQUEST(P, NZ, E, NT);
   // groups of one k1 next to each other on an XCD: they share the lines of G
   const TileId tid = xcd_tile();
   const int grp = tid.x, k1 = tid.y, m = tid.z;
@@ -354,7 +354,7 @@ k_xysplit(const cpx<P> *__restrict__ F, cpx<P> *__restrict__ G, Grid g, Split d,
   constexpr int NE = (6 * RB + NT - 1) / NT;   // last-column values per thread
   static_assert(6 * (IX - 1) <= NT && 3 * IX <= NT, "one y1 column per thread");
   static_assert(2 * RB * IX + 6 * RB <= RB * NX, "pair 0 and the last column fit the exchange rows");
-  PSG_LDS_TWIDDLES(P, NX, EPT, NT);
+  PSG_TWIDDLES_REQUEST(P, NX, EPT, NT);
   PSG_TWIDDLES_READY(P);
   cpx<P> *ex = lds, *hs = lds + RB * NX;        // exchange rows (and pair 0), pairs 1 and 2 (then the products)
   cpx<P> *last = ex + 2 * RB * IX;

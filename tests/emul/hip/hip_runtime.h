@@ -31,6 +31,10 @@
 #define __launch_bounds__(...)
 #define PSG_WAVES_PER_EU(...)
 #define PSG_FRESH(i) ((void)0)
+// the twiddles of a block in one step, for kernels whose block is a number of teams
+#define PSG_LDS_TWIDDLES(P, N, E)                  \
+  PSG_TWIDDLES_REQUEST(P, N, E, (N) / (E));        \
+  PSG_TWIDDLES_READY(P)
 #define __shared__ static thread_local
 #define PSG_DYN_SMEM(name) char *name = ::emu::dyn_smem
 #define __align__(n) __attribute__((aligned(n)))
