@@ -150,10 +150,13 @@ int psg_device_count(void);
  *  10  as 1 with registers capped for 4 waves/SIMD (FP64) or 5 (FP32-bulk)
  *  11  as 1 with registers capped for 5 waves/SIMD (FP64) or 6 (FP32-bulk)
  * x-pass of the Boussinesq right-hand side (9 inputs, 4 outputs), variants 0..11:
- *   0-4 as above; 5, 6 as 2 with 2 and 4 rows per block; 7 as 4 with 1 row per
- *   block; 8, 9 as above in FP32-bulk (in FP64: 4 points/thread, inputs per pair,
- *   2 rows per block); 10 as 2 with registers capped for 4 waves/SIMD (FP64) or 5;
- *   11 as 4 with registers capped for 5 waves/SIMD (FP64) or 6
+ *   0 the shape measured fastest for the length and precision: 8 points/thread, inputs
+ *   front-loaded, product kept for all outputs, except in the FP64 form 4 at 32 to 128
+ *   points and 3 above, in FP32-bulk 4 at 32 and 64 points and 2 at 128; 1-4 as above;
+ *   5, 6 as 2 with 2 and 4 rows per block; 7 as 4 with 1 row per block; 8, 9 as above
+ *   in FP32-bulk (in FP64: 4 points/thread, inputs per pair, 2 rows per block); 10 as 2
+ *   with registers capped for 4 waves/SIMD (FP64) or 5; 11 as 4 with registers capped
+ *   for 5 waves/SIMD (FP64) or 6
  *   (the Boussinesq flavour has no z-forward or slab variants)
  * z-forward + update pass of the 3D Navier-Stokes and Euler step (PSG_PASS_ZFWD),
  * variants 0..1:

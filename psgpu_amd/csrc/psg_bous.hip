@@ -15,86 +15,132 @@
 
 namespace psg {
 
+// The stage input Z0 and the increments X_s live in z runs (LayRun): a z-pass
+// block then reads and writes them as one run per (tile, ky), as the
+// Navier-Stokes working copy (LayW) is; the state stays in the reference order.
+typedef LayRun<4> LayZ0;
+typedef LayRun<12> LayXS;
+
 // pass 1: outputs w(3), u(3), i kx rho, i ky rho, i kz rho; with nout = 7 the
 // seventh field is rho itself (physical-space dumps, 3D_Boussinesq/src/out_low.h:79-110)
-template <typename P, int N, int T>
-__global__ void __launch_bounds__(T *(N / EPT))
+// LAY: layout of st (its field stride fs); the mask is in the reference order.
+// Gather- and register-bound: vorticity becomes velocity in its own registers,
+// in FP64 until the transforms, and every index is a constant, so that nothing
+// of a pencil lies in scratch memory and two waves share a SIMD (an earlier
+// form, with the field loop rolled, indexed its registers at run time: 400 bytes
+// of scratch a lane and one wave per SIMD; capped for three waves this one spills
+// and is slower again).  512^3 FP64 2.11 -> 1.54 ms, 256^3 0.289 -> 0.195 ms, in
+// FP32 1.91 -> 1.34 and 0.230 -> 0.165 ms.
+// SPLIT: blockIdx.z also picks vorticity, velocity or density, for grids whose
+// few blocks would run their eight transforms one after the other.
+template <typename P, int N, int T, class LAY, bool SPLIT>
+__global__ void __launch_bounds__(T *(N / EPT)) PSG_WAVES_PER_EU((N <= 512 ? 2 : 1))
 k_zinv_bous(const cpx<double> *__restrict__ st, long st_ms, long fs, cpx<P> *__restrict__ out, long out_ms, Grid g,
             const cpx<P> *__restrict__ tw, const int8_t *__restrict__ mask, int umask, int nout) {
   PSG_TWIDDLES_REQUEST(P, N, EPT, T *(N / EPT));
-  PSG_TWIDDLES_READY(P);
   constexpr int TP = N / EPT;
   const int col = threadIdx.x % T, j = threadIdx.x / T;
   const TileId tid = xcd_tile();
-  const int ikx = tid.x * T + col, iky = tid.y, m = tid.z;
+  const int ikx = tid.x * T + col, iky = tid.y, m = SPLIT ? tid.z / 3 : tid.z, part = SPLIT ? tid.z % 3 : -1;
+  const bool vort = !SPLIT || part == 0, vel = !SPLIT || part == 1, dens = !SPLIT || part == 2;
   const bool valid = ikx < g.iktx;
   const int ky = iky - g.kty;
   const double kx = (double)ikx * g.alpha, kyd = (double)ky;
   const cpx<double> *s0 = st + (long)m * st_ms;
+  cpx<P> *o = out + (long)m * out_ms;
   cpx<double> w[3][EPT];
-  double lm[EPT];
 #pragma unroll
   for (int mm = 0; mm < EPT; mm++) {
     const int kz = valid ? wrapk(j + TP * mm, g.nz, g.ktz) : PSG_NOK;
-    const FillIdx q = fill_index(g, ikx, iky, ky, kz);
-    w[0][mm] = ld_fill(s0, q);
-    w[1][mm] = ld_fill(s0 + fs, q);
-    w[2][mm] = ld_fill(s0 + 2 * fs, q);
-    lm[mm] = (umask && q.idx >= 0) ? (double)mask[q.tidx] : 1.0;
-  }
-  // i kx rho and i ky rho are one transform of rho scaled by constants of the
-  // pencil, so nine outputs take eight transforms
-#pragma unroll 1
-  for (int f = 0; f < nout; f++) {
-    cpx<P> v[EPT];
-    if (f == 7 && nout == 9) continue;   // written with field 6
-    if (f == 6) {
-      // vorticity no longer needed: reuse its registers for rho
+    const FillIdx q = fill_index<LAY>(g, ikx, iky, ky, kz);
 #pragma unroll
-      for (int mm = 0; mm < EPT; mm++) {
-        const int kz = valid ? wrapk(j + TP * mm, g.nz, g.ktz) : PSG_NOK;
-        w[0][mm] = ld_fill(s0 + 3 * fs, fill_index(g, ikx, iky, ky, kz));
-      }
+    for (int f = 0; f < 3; f++) w[f][mm] = SPLIT && part == 2 ? (f == 0 ? ld_fill(s0 + 3 * fs, q) : cpx<double>{0, 0}) : ld_fill(s0 + f * fs, q);
+  }
+  PSG_TWIDDLES_READY(P);
+  // transform one field and store it into output f
+  auto field = [&](cpx<P>(&v)[EPT], int f) {
+    fft_pencil<P, N, EPT, true>(v, lds, fresh(j), T, col, tw);
+    const int jo = fresh(j);
+    if (valid) {
+#pragma unroll
+      for (int mm = 0; mm < EPT; mm++)
+        st_pass<NT<P, PASS_ZINV>::st>(&o[(long)f * g.zsz + zoff<P>(g, ikx, iky, jo + TP * mm)], v[mm]);
     }
+  };
+  if (vort) {
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+      cpx<P> v[EPT];
+#pragma unroll
+      for (int mm = 0; mm < EPT; mm++) v[mm] = to<P>(w[f][mm]);
+      field(v, f);
+    }
+  }
+  if (vel) {
 #pragma unroll
     for (int mm = 0; mm < EPT; mm++) {
-      const int kz = wrapk(j + TP * mm, g.nz, g.ktz);
+      const int kz = valid ? wrapk(fresh(j) + TP * mm, g.nz, g.ktz) : PSG_NOK;
       const double kzd = kz == PSG_NOK ? 0.0 : (double)kz;
-      cpx<double> r;
-      if (f < 3) {
-        r = w[f][mm];
-      } else if (f < 6) {
-        const double wk = kx * kx + kyd * kyd + kzd * kzd;
-        const double wki = lm[mm] / (wk > 0.001 ? wk : 0.001);
-        cpx<double> u, vv, ww;
-        biot_savart(kx, kyd, kzd, w[0][mm], w[1][mm], w[2][mm], wki, u, vv, ww);
-        r = f == 3 ? u : (f == 4 ? vv : ww);
-      } else if (nout == 7 || f == 6) {
-        r = w[0][mm];   // rho (the gradient's x and y parts are scaled after the transform)
-      } else {
-        r = cpx<double>{-kzd * w[0][mm].y, kzd * w[0][mm].x};   // setFFK: i kz rho
+      const double wk = kx * kx + kyd * kyd + kzd * kzd;
+      double wki = 1.0;
+      if (umask) {
+        const FillIdx q = fill_index<LAY>(g, ikx, iky, ky, kz);
+        if (q.idx >= 0) wki = (double)mask[q.tidx];
       }
-      v[mm] = to<P>(r);
+      wki = wki / (wk > 0.001 ? wk : 0.001);
+      cpx<double> u, vv, ww;
+      biot_savart(kx, kyd, kzd, w[0][mm], w[1][mm], w[2][mm], wki, u, vv, ww);
+      w[0][mm] = u;
+      w[1][mm] = vv;
+      w[2][mm] = ww;
+      PSG_COMPILER_FENCE();
     }
-    fft_pencil<P, N, EPT, true>(v, lds, j, T, col, tw);
-    if (valid) {
-      cpx<P> *o = out + (long)m * out_ms + (long)f * g.zsz;
-      if (f == 6 && nout == 9) {
-        // setFFK: i kx rho and i ky rho
-        const P px = (P)kx, py = (P)kyd;
-        cpx<P> *o7 = o + g.zsz;
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+      cpx<P> v[EPT];
+#pragma unroll
+      for (int mm = 0; mm < EPT; mm++) v[mm] = to<P>(w[f][mm]);
+      // the density is requested before the last velocity transform, into
+      // registers that the vorticity has left
+      if (!SPLIT && f == 1) {
 #pragma unroll
         for (int mm = 0; mm < EPT; mm++) {
-          const long at = zoff<P>(g, ikx, iky, j + TP * mm);
-          st_pass<NT<P, PASS_ZINV>::st>(&o[at], cpx<P>{-px * v[mm].y, px * v[mm].x});
-          st_pass<NT<P, PASS_ZINV>::st>(&o7[at], cpx<P>{-py * v[mm].y, py * v[mm].x});
+          const int kz = valid ? wrapk(fresh(j) + TP * mm, g.nz, g.ktz) : PSG_NOK;
+          w[0][mm] = ld_fill(s0 + 3 * fs, fill_index<LAY>(g, ikx, iky, ky, kz));
         }
-      } else {
-#pragma unroll
-        for (int mm = 0; mm < EPT; mm++) st_pass<NT<P, PASS_ZINV>::st>(&o[zoff<P>(g, ikx, iky, j + TP * mm)], v[mm]);
       }
+      field(v, 3 + f);
     }
   }
+  if (!dens) return;
+  cpx<P> v[EPT];
+#pragma unroll
+  for (int mm = 0; mm < EPT; mm++) v[mm] = to<P>(w[0][mm]);
+  if (nout == 7) {
+    field(v, 6);
+    return;
+  }
+  // setFFK: i kx rho and i ky rho are one transform of rho scaled by constants
+  // of the pencil, so nine outputs take eight transforms
+  fft_pencil<P, N, EPT, true>(v, lds, fresh(j), T, col, tw);
+  if (valid) {
+    const int jo = fresh(j);
+    const P px = (P)kx, py = (P)kyd;
+    cpx<P> *o6 = o + 6 * g.zsz, *o7 = o6 + g.zsz;
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) {
+      const long at = zoff<P>(g, ikx, iky, jo + TP * mm);
+      st_pass<NT<P, PASS_ZINV>::st>(&o6[at], cpx<P>{-px * v[mm].y, px * v[mm].x});
+      st_pass<NT<P, PASS_ZINV>::st>(&o7[at], cpx<P>{-py * v[mm].y, py * v[mm].x});
+    }
+  }
+#pragma unroll
+  for (int mm = 0; mm < EPT; mm++) {
+    const int kz = wrapk(fresh(j) + TP * mm, g.nz, g.ktz);
+    const double kzd = kz == PSG_NOK ? 0.0 : (double)kz;
+    v[mm] = to<P>(cpx<double>{-kzd * w[0][mm].y, kzd * w[0][mm].x});   // i kz rho
+  }
+  field(v, 8);
 }
 
 // x-pass product: (U,V,W) <- -(u x w), rx <- u . grad rho  (3D_Boussinesq/src/kernels.h:298-328)
@@ -134,33 +180,36 @@ __device__ __forceinline__ void bous_rhs(const BousPar &p, double kx, double ky,
 }
 
 template <int STAGE> struct UpdBous {
-  cpx<double> *st, *s0, *xs;  // state [m][4][nkt], stage input [m][4][nkt], increments [m][3][4][nkt]
-  long nkt;
+  cpx<double> *st, *s0, *xs;  // state [m][4][nkt]; stage input (LayZ0) and increments (LayXS, field 4 stage + f)
+  long nkt, nktw;
   const int8_t *L;
   BousPar p;
-  __device__ __forceinline__ void operator()(int m, long ik, int, double kx, double ky, double kz,
+  Grid g;
+  __device__ __forceinline__ void operator()(int m, long ik, int ikx, double kx, double ky, double kz,
                                              cpx<double> (&N)[4]) const {
+    const int iky = (int)ky + g.kty, ikz = (int)kz + g.ktz;
     cpx<double> *S = st + (long)m * 4 * nkt + ik;
-    cpx<double> *Z = s0 + (long)m * 4 * nkt + ik;
-    cpx<double> *X = xs + (long)m * 12 * nkt + ik;
+    cpx<double> *Z = s0 + (long)m * 4 * nktw + LayZ0::at(g, ikx, iky, ikz);
+    cpx<double> *X = xs + (long)m * 12 * nktw + LayXS::at(g, ikx, iky, ikz);
+    constexpr int zf = 8;
     const double wk = kx * kx + ky * ky + kz * kz;
     const double dt = p.dt;
     const double LC = (double)L[ik];
     double C[8];
     if constexpr (STAGE < 3) {
-      bous_rhs(p, kx, ky, kz, LC, N, Z[0], Z[nkt], Z[2 * nkt], Z[3 * nkt], C);
+      bous_rhs(p, kx, ky, kz, LC, N, Z[0], Z[zf], Z[2 * zf], Z[3 * zf], C);
       const double q = STAGE < 2 ? 0.25 : 0.5, h = STAGE < 2 ? 0.5 : 1.0;
       const double d1 = (1. - q * dt * p.v2 * wk) / (1. + q * dt * p.v2 * wk);
       const double d2 = (1. - q * dt * p.v2 * wk / p.sc) / (1. + q * dt * p.v2 * wk / p.sc);
 #pragma unroll
       for (int f = 0; f < 4; f++) {
-        X[(STAGE * 4 + f) * nkt] = cpx<double>{dt * C[2 * f], dt * C[2 * f + 1]};
+        X[(STAGE * 4 + f) * zf] = cpx<double>{dt * C[2 * f], dt * C[2 * f + 1]};
         const double d = f < 3 ? d1 : d2;
         const cpx<double> sn = S[f * nkt];
-        Z[f * nkt] = cpx<double>{d * (sn.x + h * dt * C[2 * f]), d * (sn.y + h * dt * C[2 * f + 1])};
+        Z[f * zf] = cpx<double>{d * (sn.x + h * dt * C[2 * f]), d * (sn.y + h * dt * C[2 * f + 1])};
       }
     } else {
-      bous_rhs(p, kx, ky, kz, 1.0, N, Z[0], Z[nkt], Z[2 * nkt], Z[3 * nkt], C);
+      bous_rhs(p, kx, ky, kz, 1.0, N, Z[0], Z[zf], Z[2 * zf], Z[3 * zf], C);
       const double d1 = 1. - 0.5 * dt * p.v2 * wk, d2 = 1. - 0.5 * dt * p.v2 * wk / p.sc;
       const double den1 = 1. + 0.5 * dt * p.v2 * wk, den2 = 1. + 0.5 * dt * p.v2 * wk / p.sc;
       const double sixth = 1.0 / 6.0, third = 1.0 / 3.0;
@@ -168,10 +217,10 @@ template <int STAGE> struct UpdBous {
 #pragma unroll
       for (int f = 0; f < 4; f++) {
         const double d = f < 3 ? d1 : d2, den = f < 3 ? den1 : den2;
-        const cpx<double> sn = S[f * nkt], x1 = X[f * nkt], x2 = X[(4 + f) * nkt], x3 = X[(8 + f) * nkt];
+        const cpx<double> sn = S[f * nkt], x1 = X[f * zf], x2 = X[(4 + f) * zf], x3 = X[(8 + f) * zf];
         r[f].x = LC * (d * sn.x + sixth * (x1.x + dt * C[2 * f]) + third * (x2.x + x3.x)) / den;
         r[f].y = LC * (d * sn.y + sixth * (x1.y + dt * C[2 * f + 1]) + third * (x2.y + x3.y)) / den;
-        Z[f * nkt] = r[f];
+        Z[f * zf] = r[f];
       }
       const double wki = 1.0 / (wk > 0.001 ? wk : 0.001);
       const double phiR = (kx * r[0].y + ky * r[1].y + kz * r[2].y) * wki;
@@ -187,7 +236,7 @@ template <int STAGE> struct UpdBous {
 
 // dz/dt for Newton (3D_Boussinesq/src/kernels.h:624-692): out = -nu k^2 z + C
 struct UpdBousRHS {
-  const cpx<double> *st, *s0;
+  const cpx<double> *st;       // the state, which is also the stage input
   cpx<double> *out;
   long nkt;
   const int8_t *L;
@@ -195,9 +244,8 @@ struct UpdBousRHS {
   __device__ __forceinline__ void operator()(int m, long ik, int, double kx, double ky, double kz,
                                              cpx<double> (&N)[4]) const {
     const cpx<double> *S = st + (long)m * 4 * nkt + ik;
-    const cpx<double> *Z = s0 + (long)m * 4 * nkt + ik;
     double C[8];
-    bous_rhs(p, kx, ky, kz, (double)L[ik], N, Z[0], Z[nkt], Z[2 * nkt], Z[3 * nkt], C);
+    bous_rhs(p, kx, ky, kz, (double)L[ik], N, S[0], S[nkt], S[2 * nkt], S[3 * nkt], C);
     const double wk = kx * kx + ky * ky + kz * kz;
     const double d1 = -p.v2 * wk, d2 = -p.v2 * wk / p.sc;
     cpx<double> *o = out + (long)m * 4 * nkt + ik;
@@ -209,8 +257,15 @@ struct UpdBousRHS {
   }
 };
 
-__global__ void k_copy(const cpx<double> *__restrict__ a, cpx<double> *__restrict__ b, long n) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) b[i] = a[i];
+// stage input = state (setVelocity), in LayZ0 (padding columns zero)
+__global__ void k_stage_bous(const cpx<double> *__restrict__ a, cpx<double> *__restrict__ b, Grid g, long nktw, long total) {
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
+    const long m = i / (4 * nktw), w = i - m * 4 * nktw, run = w / 32;
+    const int f = (int)((w >> 3) & 3), ikz = (int)(run % g.iktz);
+    const long t = run / g.iktz;
+    const int iky = (int)(t % g.ikty), ikx = (int)(t / g.ikty) * 8 + (int)(w & 7);
+    b[i] = ikx < g.iktx ? a[(m * 4 + f) * g.nkt + LayNKT::at(g, ikx, iky, ikz)] : cpx<double>{0, 0};
+  }
 }
 
 // ------------------------------------------------------------------ launches
@@ -220,18 +275,24 @@ __global__ void k_copy(const cpx<double> *__restrict__ a, cpx<double> *__restric
     if (r_) return r_;  \
   } while (0)
 
-template <typename P>
-static int launch_zinv_b(Ctx *c, const cpx<double> *st, long st_ms, int umask, int nm, int nout = 9) {
+// LAY: LayZ0 (the stage input) or LayNKT (a state)
+template <typename P, class LAY>
+static int launch_zinv_b(Ctx *c, const cpx<double> *st, int umask, int nm, int nout = 9) {
   const Grid &g = c->g;
   cpx<P> *A = (cpx<P> *)c->bufA;
   PSG_DISPATCH_N(g.nz, {
     constexpr int T = Col<N, P>::T;
     dim3 grid((g.iktx + T - 1) / T, g.ikty, nm);
     size_t lds = (size_t)(N * T + N) * sizeof(cpx<P>);
-    auto k = k_zinv_bous<P, N, T>;
+    constexpr bool RUN = std::is_same<LAY, LayZ0>::value;
+    // with blocks for three quarters of the CUs or fewer: 32^3 FP64 19.4 -> 13.9 us, 64^3
+    // (129 blocks) 21.5 -> 17.0; at 128^3 (255 blocks) the split costs, 30 -> 34.3
+    const bool split = grid.x * grid.y * grid.z <= 192;
+    auto k = split ? k_zinv_bous<P, N, T, LAY, true> : k_zinv_bous<P, N, T, LAY, false>;
     PSG_HIP(lds_attr(k, lds));
-    hipLaunchKernelGGL(k, grid, dim3(Col<N, P>::THREADS), lds, c->stream, st, st_ms, g.nkt, A, 9 * g.zsz, g,
-                       twp<P>(c, 2), c->mask, umask, nout);
+    if (split) grid.z *= 3;
+    hipLaunchKernelGGL(k, grid, dim3(Col<N, P>::THREADS), lds, c->stream, st, 4 * (RUN ? c->nktw : g.nkt),
+                       RUN ? 8L : g.nkt, A, 9 * g.zsz, g, twp<P>(c, 2), c->mask, umask, nout);
   });
   PSG_HIP(hipGetLastError());
   return 0;
@@ -246,7 +307,16 @@ template <typename P> int launch_xphys(Ctx *c, const cpx<P> *in, double *out, in
 template <typename P> static int xpass_bous(Ctx *c, const cpx<P> *B, cpx<P> *Cb, int nm) {
   const long nr = (long)c->g.ny * c->g.nz;
   const ProdBous<P> pb{};
-  switch (c->xvar) {
+  // variant 0 is the shape measured fastest for the length and precision (us):
+  //   FP64, 256 points on: 3 (8 points a thread 516, this 394 at 256^3; 4530, 3543 at 512^3), 32 to 128: 4
+  //     (16.8, 14.2 at 32^3; 17.9, 15.0 at 64^3; 70.0, 60.3 at 128^3; 117, 98.8 at 64^3 with 16 members)
+  //   FP32, 32 and 64: 4 (15.8, 12.8; 15.1, 13.0), 128: 2 (37.2, 35.6), above: 8 points, product kept
+  //   16 points: 4 is faster too (19.1, 10.8), but the radix stays 8: its rounding decides
+  //     where a Newton iteration with a singular Jacobian stops on these smallest grids
+  const int n = c->g.nx;
+  const int best = n < 32 ? 0 : sizeof(P) == 8 ? (n >= 256 ? 3 : 4) : (n <= 64 ? 4 : n == 128 ? 2 : 0);
+  const int xv = c->xvar ? c->xvar : best;
+  switch (xv) {
     case 1: return launch_xpass<P, 9, 4, ProdBous<P>, 8, true, true>(c, B, Cb, nr, nm, pb);
     case 2: return launch_xpass<P, 9, 4, ProdBous<P>, 8, false, true>(c, B, Cb, nr, nm, pb);
     case 3: return launch_xpass<P, 9, 4, ProdBous<P>, 4, true, false>(c, B, Cb, nr, nm, pb);
@@ -257,7 +327,7 @@ template <typename P> static int xpass_bous(Ctx *c, const cpx<P> *B, cpx<P> *Cb,
     case 8:
     case 9:
       if constexpr (std::is_same<P, float>::value) {
-        if (c->xvar == 8) return launch_xpass<P, 9, 4, ProdBous<P>, 16, false, true>(c, B, Cb, nr, nm, pb);
+        if (xv == 8) return launch_xpass<P, 9, 4, ProdBous<P>, 16, false, true>(c, B, Cb, nr, nm, pb);
         return launch_xpass<P, 9, 4, ProdBous<P>, 16, false, true, 4>(c, B, Cb, nr, nm, pb);
       }
       return launch_xpass<P, 9, 4, ProdBous<P>, 4, false, true, 2>(c, B, Cb, nr, nm, pb);
@@ -275,7 +345,13 @@ template <typename P, class UPD> static int launch_zfwd_b(Ctx *c, const cpx<P> *
     constexpr int T = Col<N, P>::T;
     dim3 grid((g.iktx + T - 1) / T, g.ikty, nm);
     size_t lds = (size_t)(N * T + N) * sizeof(cpx<P>);
-    auto k = k_zfwd<P, N, T, 4, UPD>;
+    // short transforms: all loads of a block in flight at once, whatever the
+    // registers (up to 290 in FP64, one wave per SIMD).  From 256 points on there
+    // are blocks enough for occupancy to count: the update's loads stay within
+    // pairs of modes, and in FP64 each field is loaded at its own transform
+    // (256^3 FP64 297 -> 229 us, FP32 209 -> 201; at 64^3 it would be 21 -> 26)
+    constexpr bool LONG = N >= 256;
+    auto k = k_zfwd<P, N, T, 4, UPD, (sizeof(P) == 4 || !LONG), 1, (LONG ? 2 : 0), (LONG && N <= 512 ? 2 : 1)>;
     PSG_HIP(lds_attr(k, lds));
     hipLaunchKernelGGL(k, grid, dim3(Col<N, P>::THREADS), lds, c->stream, in, g, twp<P>(c, 2), upd);
   });
@@ -283,13 +359,13 @@ template <typename P, class UPD> static int launch_zfwd_b(Ctx *c, const cpx<P> *
   return 0;
 }
 
-template <typename P, class UPD> static int rhs_b(Ctx *c, const cpx<double> *s0, int umask, UPD upd, int nm) {
+template <typename P, class LAY, class UPD> static int rhs_b(Ctx *c, const cpx<double> *s0, int umask, UPD upd, int nm) {
   const Grid &g = c->g;
   cpx<P> *A = (cpx<P> *)c->bufA, *B = (cpx<P> *)c->bufB, *Cb = (cpx<P> *)c->bufC;
   const long Z = (long)g.iktx * g.ikty * g.nz, Y = (long)g.iktx * g.ny * g.nz;
   const long b = sizeof(cpx<P>);
   prof_begin(c, "zinv_bous", (4 * g.nkt * 16 + 9 * Z * b) * nm);
-  PSG_TRYB(launch_zinv_b<P>(c, s0, 4 * g.nkt, umask, nm));
+  PSG_TRYB((launch_zinv_b<P, LAY>(c, s0, umask, nm)));
   prof_end(c);
   prof_begin(c, "yinv", 9 * (Z + Y) * b * nm);
   PSG_TRYB(launch_yinv_g<P>(c, A, B, 9 * nm));
@@ -313,23 +389,22 @@ static BousPar bpar(const Ctx *c) {
 
 template <typename P> static int runb_t(Ctx *c, int nsteps, bool first) {
   const Grid &g = c->g;
-  const long tot = 4 * g.nkt * c->batch;
   if (first) {
     // stage input = state (setVelocity); later steps leave it equal to the state themselves
-    hipLaunchKernelGGL(k_copy, dim3((unsigned)std::min<long>(4096, (tot + 255) / 256)), dim3(256), 0, c->stream,
-                       c->state, c->stage, tot);
+    const long tot = 4 * c->nktw * c->batch;
+    hipLaunchKernelGGL(k_stage_bous, dim3((unsigned)std::min<long>(8192, (tot + 255) / 256)), dim3(256), 0, c->stream,
+                       c->state, c->stage, g, c->nktw, tot);
     PSG_HIP(hipGetLastError());
   }
   const BousPar p = bpar(c);
   for (int nt = 0; nt < nsteps; nt++) {
-    UpdBous<0> u0{c->state, c->stage, c->rh, g.nkt, c->mask, p};
-    PSG_TRYB(rhs_b<P>(c, c->stage, (first && nt == 0) ? 1 : 0, u0, c->batch));
-    UpdBous<1> u1{c->state, c->stage, c->rh, g.nkt, c->mask, p};
-    PSG_TRYB(rhs_b<P>(c, c->stage, 0, u1, c->batch));
-    UpdBous<2> u2{c->state, c->stage, c->rh, g.nkt, c->mask, p};
-    PSG_TRYB(rhs_b<P>(c, c->stage, 0, u2, c->batch));
-    UpdBous<3> u3{c->state, c->stage, c->rh, g.nkt, c->mask, p};
-    PSG_TRYB(rhs_b<P>(c, c->stage, 0, u3, c->batch));
+#define PSG_BOUS_STAGE(S)                                                                         \
+    {                                                                                             \
+      UpdBous<S> u{c->state, c->stage, c->rh, g.nkt, c->nktw, c->mask, p, g};                     \
+      PSG_TRYB((rhs_b<P, LayZ0>(c, c->stage, (S == 0 && first && nt == 0) ? 1 : 0, u, c->batch))); \
+    }
+    PSG_BOUS_STAGE(0) PSG_BOUS_STAGE(1) PSG_BOUS_STAGE(2) PSG_BOUS_STAGE(3)
+#undef PSG_BOUS_STAGE
   }
   return 0;
 }
@@ -339,13 +414,8 @@ int bous_run(Ctx *c, int nsteps, bool first) {
 }
 
 template <typename P> static int rhsb_t(Ctx *c, const cpx<double> *in, cpx<double> *out) {
-  const Grid &g = c->g;
-  // stage copy of the input (the reference's setVelocity), then one RHS
-  hipLaunchKernelGGL(k_copy, dim3((unsigned)((4 * g.nkt + 255) / 256)), dim3(256), 0, c->stream, in, c->stage,
-                     4 * g.nkt);
-  PSG_HIP(hipGetLastError());
-  UpdBousRHS u{in, c->stage, out, g.nkt, c->mask, bpar(c)};
-  return rhs_b<P>(c, c->stage, 1, u, 1);
+  UpdBousRHS u{in, out, c->g.nkt, c->mask, bpar(c)};
+  return rhs_b<P, LayNKT>(c, in, 1, u, 1);
 }
 
 int bous_timederiv(Ctx *c, const cpx<double> *in_dev, cpx<double> *out_dev) {
@@ -355,7 +425,7 @@ int bous_timederiv(Ctx *c, const cpx<double> *in_dev, cpx<double> *out_dev) {
 // physical fields of one member: w(3), u(3), rho, NR doubles each, x fastest
 template <typename P> static int physb_t(Ctx *c, const cpx<double> *st, double *out) {
   const Grid &g = c->g;
-  PSG_TRYB(launch_zinv_b<P>(c, st, 4 * g.nkt, 1, 1, 7));
+  PSG_TRYB((launch_zinv_b<P, LayNKT>(c, st, 1, 1, 7)));
   PSG_TRYB(launch_yinv_g<P>(c, (const cpx<P> *)c->bufA, (cpx<P> *)c->bufB, 7));
   return launch_xphys<P>(c, (const cpx<P> *)c->bufB, out, 7);
 }
@@ -377,10 +447,11 @@ int bous_init(Ctx *c) {
   PSG_HIP(hipMalloc(&c->bufA, c->szA));
   PSG_HIP(hipMalloc(&c->bufB, c->szB));
   PSG_HIP(hipMalloc(&c->bufC, c->szC));
-  PSG_HIP(hipMalloc(&c->rh, sizeof(cpx<double>) * 12 * g.nkt * c->batch));
-  PSG_HIP(hipMalloc(&c->stage, sizeof(cpx<double>) * 4 * g.nkt * c->batch));
-  PSG_HIP(hipMemsetAsync(c->rh, 0, sizeof(cpx<double>) * 12 * g.nkt * c->batch, c->stream));
-  PSG_HIP(hipMemsetAsync(c->stage, 0, sizeof(cpx<double>) * 4 * g.nkt * c->batch, c->stream));
+  c->nktw = (long)((g.iktx + 7) / 8) * 8 * g.ikty * g.iktz;
+  PSG_HIP(hipMalloc(&c->rh, sizeof(cpx<double>) * 12 * c->nktw * c->batch));
+  PSG_HIP(hipMalloc(&c->stage, sizeof(cpx<double>) * 4 * c->nktw * c->batch));
+  PSG_HIP(hipMemsetAsync(c->rh, 0, sizeof(cpx<double>) * 12 * c->nktw * c->batch, c->stream));
+  PSG_HIP(hipMemsetAsync(c->stage, 0, sizeof(cpx<double>) * 4 * c->nktw * c->batch, c->stream));
   return 0;
 }
 

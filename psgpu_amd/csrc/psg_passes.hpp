@@ -109,6 +109,20 @@ __device__ __forceinline__ TileId xcd_tile() {
   tws.request(tw)
 #define PSG_TWIDDLES_READY(P) tw = tws.commit(reinterpret_cast<cpx<P> *>(smem_raw))
 
+// Keep registers for data.  What depends on a thread index that has passed
+// through fresh() is computed again where it is used, instead of being moved out
+// of the loop over units or columns and held (LDS addresses, wavenumbers and
+// masks of a thread's points: hundreds of registers, spilled); the fence keeps
+// the loads of unrolled iterations from being gathered ahead of them.
+#ifndef PSG_FRESH
+#define PSG_FRESH(i) asm volatile("" : "+v"(i))
+#endif
+#define PSG_COMPILER_FENCE() asm volatile("" ::: "memory")
+__device__ __forceinline__ int fresh(int i) {
+  PSG_FRESH(i);
+  return i;
+}
+
 template <typename P> __device__ __forceinline__ cpx<P> to(cpx<double> a) { return {(P)a.x, (P)a.y}; }
 template <typename P> __device__ __forceinline__ cpx<P> to(cpx<float> a) { return {(P)a.x, (P)a.y}; }
 __device__ __forceinline__ cpx<double> up(cpx<double> a) { return a; }
@@ -250,6 +264,15 @@ struct LayW {
     return run(g, ikx, iky, ikz) * 8 + (ikx & 7);
   }
   static __device__ __forceinline__ long fs(const Grid &) { return 8; }
+};
+
+//  LayRun<F>: F fields in runs like LayW's (tables in the reference order): the
+//          Boussinesq stage input (F = 4) and its increments (F = 12)
+template <int F> struct LayRun {
+  static __device__ __forceinline__ long at(const Grid &g, int ikx, int iky, int ikz) {
+    return LayW::run(g, ikx, iky, ikz) * (F * 8) + (ikx & 7);
+  }
+  static __device__ __forceinline__ long tab(const Grid &g, int ikx, int iky, int ikz) { return LayNKT::at(g, ikx, iky, ikz); }
 };
 
 struct FillIdx {
@@ -419,8 +442,10 @@ k_yfwd(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, Grid g, const cp
 // updates always do this).
 // PIPE (with FRONT): ky rows per block, the next row's inputs requested
 // before this row's transforms (the grid's y extent is IKTY/PIPE rounded up)
-template <typename P, int N, int T, int FO, class UPD, bool FRONT = (FO <= 4), int PIPE = 1>
-__global__ void __launch_bounds__(T *(N / EPT))
+// GRP > 0: the update's loads are kept within groups of GRP modes, and the
+// registers within WPE waves per SIMD
+template <typename P, int N, int T, int FO, class UPD, bool FRONT = (FO <= 4), int PIPE = 1, int GRP = 0, int WPE = 1>
+__global__ void __launch_bounds__(T *(N / EPT)) PSG_WAVES_PER_EU(WPE)
 k_zfwd(const cpx<P> *__restrict__ in, Grid g, const cpx<P> *__restrict__ tw, UPD upd) {
   static_assert(PIPE == 1 || FRONT, "row pipelining needs front-loaded inputs");
   PSG_TWIDDLES_REQUEST(P, N, EPT, T *(N / EPT));
@@ -478,11 +503,14 @@ k_zfwd(const cpx<P> *__restrict__ in, Grid g, const cpx<P> *__restrict__ tw, UPD
       for (int mm = 0; mm < EPT; mm++) {
         const int kz = wrapk(j + TP * mm, g.nz, g.ktz);
         if (kz == PSG_NOK) continue;
-        const long ik = ((long)(kz + g.ktz) * g.ikty + iky) * g.iktx + ikx;
+        const long ik = LayNKT::at(g, ikx, iky, kz + g.ktz);
         cpx<double> nn[FO];
 #pragma unroll
         for (int f = 0; f < FO; f++) nn[f] = res[f][mm];
         upd(m, ik, ikx, kx, ky, (double)kz, nn);
+        if constexpr (GRP > 0) {
+          if (mm % GRP == GRP - 1) PSG_COMPILER_FENCE();
+        }
       }
     }
     if constexpr (PIPE > 1) {

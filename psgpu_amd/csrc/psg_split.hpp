@@ -21,23 +21,6 @@
 
 namespace psg {
 
-// Keep registers for data.  What depends on a thread index that has passed
-// through fresh() is computed again where it is used, instead of being moved out
-// of the loop over units or columns and held (LDS addresses, wavenumbers and
-// masks of a thread's points: hundreds of registers, spilled); the fence keeps
-// the loads of unrolled iterations from being gathered ahead of them.
-#ifndef PSG_FRESH
-#define PSG_FRESH(i) asm volatile("" : "+v"(i))
-#endif
-#ifndef PSG_ZS_WAVES
-#define PSG_ZS_WAVES (sizeof(P) == 4 ? 4 : 3)
-#endif
-#define PSG_COMPILER_FENCE() asm volatile("" ::: "memory")
-__device__ __forceinline__ int fresh(int i) {
-  PSG_FRESH(i);
-  return i;
-}
-
 constexpr int SPLIT_RB = 16;   // rows of the xy kernel, points of its y transform
 
 // kx columns per z-kernel block: G and F move in pieces of kb points
@@ -97,7 +80,7 @@ template <int NZ, int RA> struct ZShape {
 // their new values itself, from its own transforms (the products are real, so
 // N(-k) = conj N(k)), and must find their old values whole.
 template <typename P, int NZ, int RA>
-__global__ void __launch_bounds__((ZShape<NZ, RA>::NT)) PSG_WAVES_PER_EU(PSG_ZS_WAVES)
+__global__ void __launch_bounds__((ZShape<NZ, RA>::NT)) PSG_WAVES_PER_EU((sizeof(P) == 4 ? 4 : 3))
 k_zsplit(const cpx<P> *__restrict__ G, cpx<P> *__restrict__ F, const cpx<P> *__restrict__ st, cpx<P> *__restrict__ sn,
          cpx<P> *__restrict__ rh, const double *__restrict__ nuzn, const double *__restrict__ nu1,
          const int8_t *__restrict__ L, Grid g, Split d, const cpx<P> *__restrict__ tw, SplitUpd u) {
