@@ -194,9 +194,7 @@ int run_steps(Ctx *c, int kind, int nsteps);
 bool rec_usable(Ctx *c, double T, double dt0, int policy, int rp);
 int rec_flow(Ctx *c, const cpx<double> *in, cpx<double> *out, double T, double dt0, int policy);
 int tl_replay(Ctx *c, const cpx<double> *dz0, cpx<double> *dz1, double T, double dt0, int policy);
-int ns3d_step_rec(Ctx *c, int umask, cpx<double> *wn, cpx<double> *wstar);
-int ns3d_adjoint(Ctx *c, const cpx<double> *z0, const cpx<double> *lamT, int nsteps, int ckpt, cpx<double> *zT,
-                 cpx<double> *lam0);
+int ns3d_step_rec(Ctx *c, int umask, const cpx<double> *wn, cpx<double> *wstar, cpx<double> *next);
 int tl_alloc(Ctx *c);
 
 }  // namespace psg

@@ -31,6 +31,7 @@ template <int PHASE, bool EULER, typename R = double, typename S = double, class
   Force F;
   double dt;
   Grid g;
+  const cpx<S> *in = nullptr;  // the state the half step starts from, when it is not st itself
   __device__ __forceinline__ void operator()(int m, long ik_nkt, int ikx, double kx, double ky, double kz,
                                              cpx<double> (&N)[3]) const {
     PSG_CURL
@@ -41,6 +42,7 @@ template <int PHASE, bool EULER, typename R = double, typename S = double, class
       it = LayW::tab(g, ikx, iky, ikz);
     }
     cpx<S> *s = st + (long)m * ms + ik;
+    const cpx<S> *q = (in ? in : st) + (long)m * ms + ik;
     cpx<R> *r = rh + (long)m * ms + ik;
     const double ll = (double)L[it];
     if constexpr (PHASE == 0) {
@@ -48,7 +50,7 @@ template <int PHASE, bool EULER, typename R = double, typename S = double, class
         r[0] = to<R>(cpx<double>{ll * xiX, ll * xiY});
         r[fs] = to<R>(cpx<double>{ll * etX, ll * etY});
         r[2 * fs] = to<R>(cpx<double>{ll * ztX, ll * ztY});
-        const cpx<double> a = up(s[0]), b = up(s[fs]), c = up(s[2 * fs]);
+        const cpx<double> a = up(q[0]), b = up(q[fs]), c = up(q[2 * fs]);
         s[0] = to<S>(cpx<double>{a.x + dt * xiX, a.y + dt * xiY});
         s[fs] = to<S>(cpx<double>{b.x + dt * etX, b.y + dt * etY});
         s[2 * fs] = to<S>(cpx<double>{c.x + dt * ztX, c.y + dt * ztY});
@@ -59,7 +61,7 @@ template <int PHASE, bool EULER, typename R = double, typename S = double, class
         r[0] = to<R>(cpx<double>{xiX, xiY});
         r[fs] = to<R>(cpx<double>{etX, etY});
         r[2 * fs] = to<R>(cpx<double>{ztX, ztY});
-        const cpx<double> a = up(s[0]), b = up(s[fs]), c = up(s[2 * fs]);
+        const cpx<double> a = up(q[0]), b = up(q[fs]), c = up(q[2 * fs]);
         s[0] = to<S>(cpx<double>{NU1 * (NUZN * a.x + xiX), NU1 * (NUZN * a.y + xiY)});
         s[fs] = to<S>(cpx<double>{NU1 * (NUZN * b.x + etX), NU1 * (NUZN * b.y + etY)});
         s[2 * fs] = to<S>(cpx<double>{NU1 * (NUZN * c.x + ztX), NU1 * (NUZN * c.y + ztY)});
@@ -71,7 +73,7 @@ template <int PHASE, bool EULER, typename R = double, typename S = double, class
         NU2 = 0.5 * nu1[it];
         add_forcing(F, kx, ky, kz, xiX, etY, ztX, ztY);
       }
-      const cpx<double> a = up(s[0]), b = up(s[fs]), c = up(s[2 * fs]);
+      const cpx<double> a = up(q[0]), b = up(q[fs]), c = up(q[2 * fs]);
       const cpx<double> ra = up(r[0]), rb = up(r[fs]), rc = up(r[2 * fs]);
       s[0] = to<S>(cpx<double>{ll * (a.x + NU2 * (xiX - ra.x)), ll * (a.y + NU2 * (xiY - ra.y))});
       s[fs] = to<S>(cpx<double>{ll * (b.x + NU2 * (etX - rb.x)), ll * (b.y + NU2 * (etY - rb.y))});
@@ -399,24 +401,23 @@ int ns3d_run(Ctx *c, int nsteps, bool first) {
 // One Navier-Stokes step of member 0 that records w^n (before the step) and
 // the predictor state w* into wn / wstar (device, 3*nkt complex each, either
 // may be null): the trajectory the adjoint sweep of a checkpoint segment needs.
-template <typename P> static int step_rec_t(Ctx *c, int umask, cpx<double> *wn, cpx<double> *wstar) {
+template <typename P>
+static int step_rec_t(Ctx *c, int umask, const cpx<double> *wn, cpx<double> *wstar, cpx<double> *next) {
   const Grid &g = c->g;
   Force F{c->cfg.force, c->cfg.kf, c->cfg.ampfor};
   const long ms = 3 * g.nkt, fs = g.nkt;
-  const size_t bytes = sizeof(cpx<double>) * 3 * g.nkt;
-  if (wn) PSG_HIP(hipMemcpyAsync(wn, c->state, bytes, hipMemcpyDeviceToDevice, c->stream));
   const long sb = (6 * 16 + 3 * (long)sizeof(cpx<P>)) * g.nkt;
-  UpdHeun<0, false, P> up{c->state, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g};
-  PSG_TRY(rhs3<P>(c, c->state, ms, umask, up, sb, 1));
-  if (wstar) PSG_HIP(hipMemcpyAsync(wstar, c->state, bytes, hipMemcpyDeviceToDevice, c->stream));
-  UpdHeun<1, false, P> uc{c->state, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g};
-  PSG_TRY(rhs3<P>(c, c->state, ms, 0, uc, sb, 1));
+  UpdHeun<0, false, P> up{wstar, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g, wn};
+  PSG_TRY(rhs3<P>(c, wn, ms, umask, up, sb, 1));
+  if (!next) return 0;
+  UpdHeun<1, false, P> uc{next, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g, wstar};
+  PSG_TRY(rhs3<P>(c, wstar, ms, 0, uc, sb, 1));
   return 0;
 }
 
-int ns3d_step_rec(Ctx *c, int umask, cpx<double> *wn, cpx<double> *wstar) {
-  return c->cfg.precision == PSG_FP32BULK ? step_rec_t<float>(c, umask, wn, wstar)
-                                          : step_rec_t<double>(c, umask, wn, wstar);
+int ns3d_step_rec(Ctx *c, int umask, const cpx<double> *wn, cpx<double> *wstar, cpx<double> *next) {
+  return c->cfg.precision == PSG_FP32BULK ? step_rec_t<float>(c, umask, wn, wstar, next)
+                                          : step_rec_t<double>(c, umask, wn, wstar, next);
 }
 
 template <typename P> static int nonlin_t(Ctx *c, const cpx<double> *in, cpx<double> *out) {

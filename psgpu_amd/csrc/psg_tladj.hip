@@ -19,9 +19,9 @@
 // (9 inverse fields w, u, G; 6 forward fields), and the step transposes to
 //   l*  = L (l' + C'(w*)^T (NU1/2 l'))
 //   l   = L (NU1 NUZN l* + C'(w)^T (NU1 (l* - l'/2)))
-// The adjoint sweep over n steps keeps a checkpoint every `ckpt` steps and
-// recomputes each segment forward, recording w^n and w*, before sweeping it
-// backward.
+// The adjoint sweep over n steps keeps a checkpoint every `ckpt` steps, records
+// w^n and w* of the last segment as it integrates, recomputes and records each
+// earlier segment, and sweeps every segment backward.
 #include "psg_ns3d.hpp"
 #include "../../include/psg_adjoint.h"
 #include <algorithm>
@@ -258,130 +258,116 @@ static int rhs_adj(Ctx *c, const cpx<double> *w, const cpx<double> *v, const dou
   return 0;
 }
 
-__global__ void k_mask_copy(const cpx<double> *__restrict__ a, cpx<double> *__restrict__ b,
-                            const int8_t *__restrict__ L, long nkt, long n) {
+__global__ void k_mask_state(cpx<double> *__restrict__ a, const int8_t *__restrict__ L, long nkt, long n) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     const double l = (double)L[i % nkt];
     const cpx<double> v = a[i];
-    b[i] = cpx<double>{l * v.x, l * v.y};
+    a[i] = cpx<double>{l * v.x, l * v.y};
   }
 }
 
-// masked copy of z0 into member 0, then nsteps recorded steps, keeping a
-// checkpoint every K steps in ck (when not null)
-static int fwd_masked(Ctx *c, const cpx<double> *z0, int nsteps, cpx<double> *ck, int K) {
-  const Grid &g = c->g;
-  const long n3 = 3 * g.nkt;
-  const size_t sb = sizeof(cpx<double>) * n3;
-  const unsigned nb = (unsigned)std::min<long>(2048, (n3 + 255) / 256);
-  hipLaunchKernelGGL(k_mask_copy, dim3(nb), dim3(256), 0, c->stream, z0, c->state, c->mask, g.nkt, n3);
-  PSG_HIP(hipGetLastError());
-  for (int n = 0; n < nsteps; n++) {
-    if (ck && n % K == 0)
-      PSG_HIP(hipMemcpyAsync(ck + (long)(n / K) * n3, c->state, sb, hipMemcpyDeviceToDevice, c->stream));
-    PSG_TRY(ns3d_step_rec(c, n == 0 ? 1 : 0, nullptr, nullptr));
-  }
-  return 0;
-}
-
-template <typename P>
-static int adjoint_t(Ctx *c, const cpx<double> *z0, const cpx<double> *lamT, int nsteps, int K, cpx<double> *zT,
-                     cpx<double> *lam0) {
-  const Grid &g = c->g;
-  const long n3 = 3 * g.nkt;
-  const size_t sb = sizeof(cpx<double>) * n3;
-  const int nck = (nsteps + K - 1) / K;
-  cpx<double> *ck = nullptr, *traj = nullptr, *lam = nullptr, *lstar = nullptr, *nuv = nullptr, *fin = nullptr;
-  int r = 0;
-  auto cleanup = [&]() {
+// One adjoint sweep: n steps in segments of K, the recorded w^n, w* of one
+// segment (slots 2i, 2i+1 of traj) and the states that the others start from.
+// Every half step reads one buffer and writes another, so that recording costs no
+// copies.  The last segment is recorded as the forward sweep runs through it and
+// is not integrated again, and a recomputed segment ends with its last w*: for 20
+// steps in two segments 99 right-hand sides instead of 120 (at 128^3 105 us each,
+// and 1.4 ms of copies a sweep: 21.8 -> 18.0 ms).
+struct Sweep {
+  Ctx *c;
+  int n, K, nseg;
+  long n3;
+  cpx<double> *buf = nullptr;
+  ~Sweep() {
+    if (!buf) return;
     (void)hipStreamSynchronize(c->stream);
-    for (cpx<double> *p : {ck, traj, lam, lstar, nuv, fin})
-      if (p) (void)hipFree(p);
-  };
-#define PSG_ADJ_TRY(x)             \
-  do {                             \
-    if ((r = (x))) { cleanup(); return r; } \
-  } while (0)
-#define PSG_ADJ_HIP(x)                                                             \
-  do {                                                                             \
-    hipError_t e_ = (x);                                                           \
-    if (e_ != hipSuccess) {                                                        \
-      set_error("%s failed: %s", #x, hipGetErrorString(e_));                       \
-      cleanup();                                                                   \
-      return PSG_EHIP;                                                             \
-    }                                                                              \
-  } while (0)
-  PSG_ADJ_HIP(hipMalloc(&ck, sb * (size_t)nck));
-  PSG_ADJ_HIP(hipMalloc(&traj, sb * 2 * (size_t)K));
-  PSG_ADJ_HIP(hipMalloc(&lam, sb));
-  PSG_ADJ_HIP(hipMalloc(&lstar, sb));
-  PSG_ADJ_HIP(hipMalloc(&nuv, sb));
-  PSG_ADJ_HIP(hipMalloc(&fin, sb));
-  const unsigned nb = (unsigned)std::min<long>(2048, (n3 + 255) / 256);
-  // forward sweep from the masked initial state, keeping checkpoints
-  PSG_ADJ_TRY(fwd_masked(c, z0, nsteps, ck, K));
-  PSG_ADJ_HIP(hipMemcpyAsync(fin, c->state, sb, hipMemcpyDeviceToDevice, c->stream));
-  if (zT) PSG_ADJ_HIP(hipMemcpyAsync(zT, fin, sb, hipMemcpyDeviceToDevice, c->stream));
-  hipLaunchKernelGGL(k_mask_copy, dim3(nb), dim3(256), 0, c->stream, lamT, lam, c->mask, g.nkt, n3);
-  PSG_ADJ_HIP(hipGetLastError());
-  // backward sweep, one checkpoint segment at a time
-  for (int s = nck - 1; s >= 0; s--) {
-    const int n0 = s * K, n1 = std::min(nsteps, n0 + K);
-    PSG_ADJ_HIP(hipMemcpyAsync(c->state, ck + (long)s * n3, sb, hipMemcpyDeviceToDevice, c->stream));
-    for (int n = n0; n < n1; n++)
-      PSG_ADJ_TRY(ns3d_step_rec(c, n == 0 ? 1 : 0, traj + (long)(2 * (n - n0)) * n3,
-                                traj + (long)(2 * (n - n0) + 1) * n3));
-    for (int n = n1 - 1; n >= n0; n--) {
-      const cpx<double> *wn = traj + (long)(2 * (n - n0)) * n3, *ws = traj + (long)(2 * (n - n0) + 1) * n3;
-      UpdAdj<0> a0{lam, lstar, nuv, g.nkt, c->nuzn, c->nu1, c->mask};
-      PSG_ADJ_TRY(rhs_adj<P>(c, ws, lam, c->nu1, 0.5, a0));
-      UpdAdj<1> a1{lam, lstar, nuv, g.nkt, c->nuzn, c->nu1, c->mask};
-      PSG_ADJ_TRY(rhs_adj<P>(c, wn, nuv, nullptr, 1.0, a1));
+    (void)hipFree(buf);
+  }
+  cpx<double> *slot(long i) const { return buf + i * n3; }
+  cpx<double> *traj(int i) const { return slot(i); }
+  cpx<double> *lam() const { return slot(2L * K); }
+  cpx<double> *lstar() const { return slot(2L * K + 1); }
+  cpx<double> *nuv() const { return slot(2L * K + 2); }
+  // the state that segment s starts from
+  cpx<double> *start(int s) const { return s == nseg - 1 ? traj(0) : slot(2L * K + 3 + s); }
+  int masked(cpx<double> *a) const {
+    const unsigned nb = (unsigned)std::min<long>(2048, (n3 + 255) / 256);
+    hipLaunchKernelGGL(k_mask_state, dim3(nb), dim3(256), 0, c->stream, a, c->mask, c->g.nkt, n3);
+    PSG_HIP(hipGetLastError());
+    return 0;
+  }
+  int open(Ctx *ctx, int nsteps, int ckpt) {
+    c = ctx;
+    if (c->cfg.flavour != PSG_NS3D) {
+      set_error("3D adjoint: Navier-Stokes flavour only");
+      return PSG_EINVAL;
     }
+    if (nsteps < 1 || ckpt < 1) {
+      set_error("adjoint: nsteps and ckpt must be >= 1");
+      return PSG_EINVAL;
+    }
+    if (int r = tl_alloc(c)) return r;
+    n = nsteps;
+    K = std::min(ckpt, nsteps);
+    nseg = (n + K - 1) / K;
+    n3 = 3 * c->g.nkt;
+    const size_t bytes = sizeof(cpx<double>) * n3 * (2 * (size_t)K + 3 + nseg - 1);
+    if (hipMalloc(&buf, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      buf = nullptr;
+      set_error("hipMalloc of %zu bytes failed", bytes);
+      return PSG_ENOMEM;
+    }
+    return 0;
   }
-  PSG_ADJ_HIP(hipMemcpyAsync(lam0, lam, sb, hipMemcpyDeviceToDevice, c->stream));
-  // leave the context holding Phi(z0), as after a forward run
-  PSG_ADJ_HIP(hipMemcpyAsync(c->state, fin, sb, hipMemcpyDeviceToDevice, c->stream));
-#undef PSG_ADJ_TRY
-#undef PSG_ADJ_HIP
-  cleanup();
-  return 0;
-}
-
-int ns3d_adjoint(Ctx *c, const cpx<double> *z0, const cpx<double> *lamT, int nsteps, int ckpt, cpx<double> *zT,
-                 cpx<double> *lam0) {
-  if (c->cfg.flavour != PSG_NS3D) {
-    set_error("3D adjoint: Navier-Stokes flavour only");
-    return PSG_EINVAL;
+  // masked z0 (host) through n steps; c->state is left holding Phi(z0)
+  int forward(const double *z0) {
+    PSG_HIP(hipMemcpyAsync(start(0), z0, sizeof(cpx<double>) * n3, hipMemcpyHostToDevice, c->stream));
+    if (int r = masked(start(0))) return r;
+    for (int s = 0; s < nseg; s++) {
+      const bool rec = s == nseg - 1;
+      const int n0 = s * K, n1 = std::min(n, n0 + K);
+      for (int i = n0; i < n1; i++) {
+        const cpx<double> *w = rec ? traj(2 * (i - n0)) : i == n0 ? start(s) : c->state;
+        cpx<double> *next = i + 1 == n ? c->state : rec ? traj(2 * (i - n0) + 2) : i + 1 == n1 ? start(s + 1) : c->state;
+        PSG_TRY(ns3d_step_rec(c, i == 0 ? 1 : 0, w, rec ? traj(2 * (i - n0) + 1) : c->state, next));
+      }
+    }
+    return 0;
   }
-  if (nsteps < 1 || ckpt < 1) {
-    set_error("adjoint: nsteps and ckpt must be >= 1");
-    return PSG_EINVAL;
+  // lam() (masked here) from the end of the sweep to its start
+  template <typename P> int backward_t() {
+    if (int r = masked(lam())) return r;
+    for (int s = nseg - 1; s >= 0; s--) {
+      const int n0 = s * K, n1 = std::min(n, n0 + K);
+      // w^n of the i-th step of the segment
+      auto wn = [&](int i) { return i == 0 ? start(s) : traj(2 * i); };
+      if (s < nseg - 1)
+        for (int i = 0; i < n1 - n0; i++)
+          PSG_TRY(ns3d_step_rec(c, n0 + i == 0 ? 1 : 0, wn(i), traj(2 * i + 1), i + 1 < n1 - n0 ? wn(i + 1) : nullptr));
+      for (int i = n1 - n0 - 1; i >= 0; i--) {
+        UpdAdj<0> a0{lam(), lstar(), nuv(), c->g.nkt, c->nuzn, c->nu1, c->mask};
+        PSG_TRY(rhs_adj<P>(c, traj(2 * i + 1), lam(), c->nu1, 0.5, a0));
+        UpdAdj<1> a1{lam(), lstar(), nuv(), c->g.nkt, c->nuzn, c->nu1, c->mask};
+        PSG_TRY(rhs_adj<P>(c, wn(i), nuv(), nullptr, 1.0, a1));
+      }
+    }
+    return 0;
   }
-  if (int r = tl_alloc(c)) return r;
-  return c->cfg.precision == PSG_FP32BULK ? adjoint_t<float>(c, z0, lamT, nsteps, ckpt, zT, lam0)
-                                          : adjoint_t<double>(c, z0, lamT, nsteps, ckpt, zT, lam0);
-}
+  // lam0 (host) = Phi'^T lamT (host)
+  int backward(const double *lamT, double *lam0) {
+    const size_t sb = sizeof(cpx<double>) * n3;
+    PSG_HIP(hipMemcpyAsync(lam(), lamT, sb, hipMemcpyHostToDevice, c->stream));
+    if (int r = c->cfg.precision == PSG_FP32BULK ? backward_t<float>() : backward_t<double>()) return r;
+    PSG_HIP(hipMemcpyAsync(lam0, lam(), sb, hipMemcpyDeviceToHost, c->stream));
+    return 0;
+  }
+};
 
 }  // namespace psg
 
 // ------------------------------------------------------------------ C-ABI
 using namespace psg;
-
-namespace {
-// host staging of nf*nkt complex arrays for one member
-struct Dev {
-  cpx<double> *p = nullptr;
-  ~Dev() { if (p) (void)hipFree(p); }
-};
-int dev_alloc(Dev &d, size_t bytes) {
-  if (hipMalloc(&d.p, bytes) != hipSuccess) {
-    set_error("hipMalloc of %zu bytes failed", bytes);
-    return PSG_ENOMEM;
-  }
-  return 0;
-}
-}  // namespace
 
 extern "C" {
 
@@ -402,17 +388,11 @@ int psg_tangent_steps(psg_ctx *c, const double *z0, const double *dz0, int nstep
 int psg_adjoint(psg_ctx *c, const double *z0, const double *lamT, int nsteps, int ckpt, double *zT, double *lam0) {
   if (!c || !z0 || !lamT || !lam0) { set_error("psg_adjoint: bad argument"); return PSG_EINVAL; }
   if (c->g.dim != 3) { set_error("psg_adjoint: 3D Navier-Stokes only"); return PSG_EINVAL; }
-  const size_t sb = sizeof(cpx<double>) * 3 * c->g.nkt;
-  Dev dz, dl, dzT, dl0;
-  if (int r = dev_alloc(dz, sb)) return r;
-  if (int r = dev_alloc(dl, sb)) return r;
-  if (int r = dev_alloc(dzT, sb)) return r;
-  if (int r = dev_alloc(dl0, sb)) return r;
-  PSG_HIP(hipMemcpyAsync(dz.p, z0, sb, hipMemcpyHostToDevice, c->stream));
-  PSG_HIP(hipMemcpyAsync(dl.p, lamT, sb, hipMemcpyHostToDevice, c->stream));
-  if (int r = ns3d_adjoint(c, dz.p, dl.p, nsteps, ckpt, dzT.p, dl0.p)) return r;
-  if (zT) PSG_HIP(hipMemcpyAsync(zT, dzT.p, sb, hipMemcpyDeviceToHost, c->stream));
-  PSG_HIP(hipMemcpyAsync(lam0, dl0.p, sb, hipMemcpyDeviceToHost, c->stream));
+  Sweep w;
+  if (int r = w.open(c, nsteps, ckpt)) return r;
+  if (int r = w.forward(z0)) return r;
+  if (zT) PSG_HIP(hipMemcpyAsync(zT, c->state, sizeof(cpx<double>) * w.n3, hipMemcpyDeviceToHost, c->stream));
+  if (int r = w.backward(lamT, lam0)) return r;
   PSG_HIP(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -423,21 +403,16 @@ int psg_residual_grad(psg_ctx *c, const double *z0, int nsteps, int ckpt, double
   if (c->g.dim != 3) { set_error("psg_residual_grad: 3D Navier-Stokes only"); return PSG_EINVAL; }
   const Grid &g = c->g;
   const long nkt = g.nkt;
+  if (c->cfg.flavour != PSG_NS3D) { set_error("psg_residual_grad: Navier-Stokes flavour only"); return PSG_EINVAL; }
   std::vector<int8_t> L(nkt);
   PSG_HIP(hipMemcpy(L.data(), c->mask, nkt, hipMemcpyDeviceToHost));
   std::vector<double> fin(6 * nkt), r(6 * nkt), lam0(6 * nkt);
   {
-    const size_t sb = sizeof(cpx<double>) * 3 * nkt;
-    Dev dz, dzT, dl, dl0;
-    if (int e = dev_alloc(dz, sb)) return e;
-    if (int e = dev_alloc(dzT, sb)) return e;
-    if (int e = dev_alloc(dl, sb)) return e;
-    if (int e = dev_alloc(dl0, sb)) return e;
-    PSG_HIP(hipMemcpyAsync(dz.p, z0, sb, hipMemcpyHostToDevice, c->stream));
-    // residual r = Phi(z0) - S z0 needs Phi(z0) first: the same masked forward sweep
-    if (c->cfg.flavour != PSG_NS3D) { set_error("psg_residual_grad: Navier-Stokes flavour only"); return PSG_EINVAL; }
-    if (int e = fwd_masked(c, dz.p, nsteps, nullptr, 1)) return e;
-    PSG_HIP(hipMemcpyAsync(fin.data(), c->state, sb, hipMemcpyDeviceToHost, c->stream));
+    Sweep w;
+    if (int e = w.open(c, nsteps, ckpt)) return e;
+    // the residual r = Phi(z0) - S z0 needs Phi(z0) first
+    if (int e = w.forward(z0)) return e;
+    PSG_HIP(hipMemcpyAsync(fin.data(), c->state, sizeof(double) * 6 * nkt, hipMemcpyDeviceToHost, c->stream));
     PSG_HIP(hipStreamSynchronize(c->stream));
     double Jv = 0.0;
     for (long f = 0; f < 3; f++)
@@ -454,9 +429,7 @@ int psg_residual_grad(psg_ctx *c, const double *z0, int nsteps, int ckpt, double
         Jv += rr * rr + ri * ri;
       }
     *J = Jv;
-    PSG_HIP(hipMemcpyAsync(dl.p, r.data(), sb, hipMemcpyHostToDevice, c->stream));
-    if (int e = ns3d_adjoint(c, dz.p, dl.p, nsteps, ckpt, dzT.p, dl0.p)) return e;
-    PSG_HIP(hipMemcpyAsync(lam0.data(), dl0.p, sb, hipMemcpyDeviceToHost, c->stream));
+    if (int e = w.backward(r.data(), lam0.data())) return e;
     PSG_HIP(hipStreamSynchronize(c->stream));
   }
   // grad = Phi'^T (2r) - S^{-1} (2r)
