@@ -247,7 +247,13 @@ static int rhs_adj(Ctx *c, const cpx<double> *w, const cpx<double> *v, const dou
   PSG_TRY(launch_yinv_g<P>(c, A, B, 9));
   prof_end(c);
   prof_begin(c, "adj_xpass", pb[2]);
-  PSG_TRY((launch_xpass<P, 9, 6, ProdNSAdj<P>, 4, false>(c, B, Cb, (long)g.ny * g.nz, 1, ProdNSAdj<P>{})));
+  // from 128 points the 15 transforms are bound by what a thread keeps in flight: 8 points
+  // a thread, all inputs requested first, the product evaluated again per output pair
+  // (us, against 4 points a thread: 128^3 57 and 68, 256^3 403 and 483, FP32-bulk 41 and
+  // 42, 246 and 292); shorter rows leave too few threads so (64^3: 19 and 16)
+  const long nr = (long)g.ny * g.nz;
+  if (g.nx >= 128) PSG_TRY((launch_xpass<P, 9, 6, ProdNSAdj<P>, 8, true, true>(c, B, Cb, nr, 1, ProdNSAdj<P>{})));
+  else PSG_TRY((launch_xpass<P, 9, 6, ProdNSAdj<P>, 4, false>(c, B, Cb, nr, 1, ProdNSAdj<P>{})));
   prof_end(c);
   prof_begin(c, "adj_yfwd", pb[3]);
   PSG_TRY(launch_yfwd_g<P>(c, Cb, A, 6));
