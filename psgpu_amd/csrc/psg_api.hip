@@ -273,10 +273,12 @@ static void free_ctx(Ctx *c) {
   void *ptrs[] = {c->state, c->rh, c->stage, c->tmp, c->st32, c->stw, c->wnuzn, c->wnu1, c->wmask, c->nuzn, c->nu1, c->nu, c->mask, c->tl_state, c->tl_stage,
                   c->tl_rh, c->tl_bufA, c->tl_bufB, c->tl_bufC, c->bufA, c->bufB, c->bufC,
                   c->tw64[0], c->tw64[1], c->tw64[2], c->tw32[0], c->tw32[1], c->tw32[2], c->dred, c->io, c->dtm,
-                  c->rec, c->rec_cnt};
+                  c->rec, c->rec_cnt, c->adj};
   for (void *p : ptrs)
     if (p) hipFree(p);
   for (auto e : c->evs) hipEventDestroy(e);
+  if (c->copy_ev) hipEventDestroy(c->copy_ev);
+  if (c->copy_stream) hipStreamDestroy(c->copy_stream);
   if (c->stream) hipStreamDestroy(c->stream);
 }
 

@@ -86,6 +86,12 @@ struct Ctx {
   cpx<double> *tl_state = nullptr, *tl_stage = nullptr, *tl_rh = nullptr;
   bool tl_fp32 = false;             // tangent-linear passes in FP32-bulk in an FP64 context
   void *tl_bufA = nullptr, *tl_bufB = nullptr, *tl_bufC = nullptr;
+  // adjoint sweep: recorded states and work fields, kept up to 1 GiB (a gradient
+  // descent sweeps again and again), and the stream of its host copies
+  cpx<double> *adj = nullptr;
+  size_t adj_bytes = 0;
+  hipStream_t copy_stream = nullptr;
+  hipEvent_t copy_ev = nullptr;
   // 2D recorded base trajectory: the physical (w, u, v) of every RK stage of
   // one base flow, [slot = 4 step + stage][field][y][x] in rec_p bytes per
   // value (8, or 4 for FP32 tangent-linear passes); rec_cnt is the device
