@@ -255,13 +255,17 @@ static int launch_xpass2(Ctx *c, const cpx<P> *in, cpx<P> *out, long nrow_m, int
       hipLaunchKernelGGL(k, dim3((unsigned)nrows), dim3(NT), lds, c->stream, in, out, nrow_m, nrows, g,
                          twp<P>(c, 0), prod);
     } else {
-      constexpr int TE = Row<N>::TEAMS;
-      dim3 grid((unsigned)((nrows + TE - 1) / TE));
-      size_t lds = (size_t)(row_len<N>() * TE + N) * sizeof(cpx<P>);
-      auto k = k_xpass<P, N, TE, FI, FO, PROD, EPT, true, false, 0, YCol>;
+      // rows per block: pieces of 64 bytes from 512 points on, lines below.  Twice the rows
+      // leaves one or two blocks a CU, whose barriers then stand alone (FP64 us, this and
+      // twice: 512^2 x 8 23.6, 27.3; 1024^2 x 4 48.1, 64.3); half of them in FP32 gathers
+      // 32 bytes (FP32 512^2 x 8 15.3, 15.8; 1024^2 x 2 20.3, 21.7)
+      constexpr int TE = Row<N>::TEAMS * (sizeof(P) == 4 && N >= 512 ? 2 : 1);
+      constexpr size_t lds = xcol_lds<P, N, TE>();
+      static_assert(TE * Row<N>::TPX <= 1024 && lds <= 160 * 1024, "column x-pass block size");
+      auto k = k_xpass_col<P, N, TE, FI, FO, PROD>;
       PSG_HIP(lds_attr(k, lds));
-      hipLaunchKernelGGL(k, grid, dim3(Row<N>::THREADS), lds, c->stream, in, out, nrow_m, nrows, g,
-                         twp<P>(c, 0), prod, 0);
+      hipLaunchKernelGGL(k, dim3((unsigned)((nrows + TE - 1) / TE)), dim3(TE * Row<N>::TPX), lds, c->stream, in, out,
+                         nrow_m, nrows, g, twp<P>(c, 0), prod);
     }
   });
   PSG_HIP(hipGetLastError());

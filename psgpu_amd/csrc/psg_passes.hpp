@@ -580,7 +580,7 @@ __device__ __forceinline__ void split_pair(cpx<P> zk, cpx<P> zc, cpx<P> &A, cpx<
 // WPE > 0 asks the compiler for at least WPE waves per SIMD (a register cap
 // of 512/WPE VGPRs), trading spills or rematerialisation for occupancy.
 template <typename P, int N, int TEAMS, int FI, int FO, class PROD, int E = EPT, bool FRONT = true,
-          bool LAZY = false, int WPE = 0, class YL = YTile<P>>
+          bool LAZY = false, int WPE = 0>
 __global__ void __launch_bounds__(TEAMS *(N / E)) PSG_WAVES_PER_EU(WPE > 0 ? WPE : 1)
 k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, long nrows, Grid g,
         const cpx<P> *__restrict__ tw, PROD prod, int zs0) {
@@ -593,8 +593,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   // row = (m, z, y) with y fastest over the launch's planes zs0 .. zs0 +
   // nrow_m/ny - 1 of each member: the block's first row is split once per
   // block (uniform), each team steps y from it (launches keep nrows < 2^31)
-  const unsigned blk = std::is_same<YL, YCol>::value ? (unsigned)xcd_tile().x : blockIdx.x;
-  const unsigned row0 = blk * (unsigned)TEAMS, nrm = (unsigned)nrow_m, ny = (unsigned)g.ny;
+  const unsigned row0 = blockIdx.x * (unsigned)TEAMS, nrm = (unsigned)nrow_m, ny = (unsigned)g.ny;
   const unsigned m0 = row0 / nrm, rr0 = row0 - m0 * nrm, z0 = rr0 / ny, nzr = nrm / ny;
   unsigned y = rr0 - z0 * ny + team, z = z0, m = m0;
   while (y >= ny) { y -= ny; z++; }
@@ -606,7 +605,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   cpx<P> *tl = lds + team * row_len<N>();
   constexpr int SW = row_swizzle<E>();
   constexpr int ix = xband<N>();
-  const long ro = YL::row(g, (int)y, (int)z);
+  const long ro = YTile<P>::row(g, (int)y, (int)z);
   auto rowp = [&](int f) { return in + ((long)m * FI + f) * g.ysz + ro; };
   // nine front-loaded fields leave no registers for the twiddles' trip (the
   // FP32 256-point Boussinesq pass ran 0.5% slower with it)
@@ -616,8 +615,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   if constexpr (FRONT) {
 #pragma unroll
     for (int p = 0; p < PI; p++)
-      XRow<P, N, E, YL>::load(vin[p], rowp(2 * p), rowp(2 * p + 1 < FI ? 2 * p + 1 : 2 * p), 2 * p + 1 < FI, valid, j,
-                          g);
+      XRow<P, N, E>::load(vin[p], rowp(2 * p), rowp(2 * p + 1 < FI ? 2 * p + 1 : 2 * p), 2 * p + 1 < FI, valid, j, g);
   }
   if constexpr (!TWFIRST) PSG_TWIDDLES_READY(P);
   P phys[2 * PI][E];
@@ -629,7 +627,7 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
 #pragma unroll
       for (int mm = 0; mm < E; mm++) v[mm] = vin[p][mm];
     } else {
-      XRow<P, N, E, YL>::load(v, rowp(fa), rowp(fb < FI ? fb : fa), fb < FI, valid, j, g);
+      XRow<P, N, E>::load(v, rowp(fa), rowp(fb < FI ? fb : fa), fb < FI, valid, j, g);
     }
     fft_pencil<P, N, E, true, WAVE, SW>(v, tl, j, 1, 0, tw);
 #pragma unroll
@@ -675,35 +673,119 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
       const int k = j + TPX * mm;   // only the kept modes and their mirrors are read back
       if (k < ix || k > N - ix) tl[lpos<SW>(k)] = v[mm];
     }
-    if constexpr (std::is_same<YL, YCol>::value) {
-      // columns of C: the block's rows lie next to each other in a column, so
-      // its threads take (kx, row) with the row fastest
-      __syncthreads();
-      constexpr int NTH = TEAMS * TPX;
-      for (int i = threadIdx.x; i < ix * TEAMS; i += NTH) {
-        const int r = i % TEAMS, k = i / TEAMS;
-        const unsigned rw = row0 + r, mr = rw / nrm;
-        if (rw < (unsigned long)nrows) {
-          const cpx<P> *tr = lds + r * row_len<N>();
-          cpx<P> A, B;
-          split_pair(tr[lpos<SW>(k)], tr[lpos<SW>((N - k) & (N - 1))], A, B);
-          cpx<P> *o = out + ((long)mr * FO + 2 * q) * g.ysz + YL::col(g, k) + (rw - mr * nrm);
-          o[0] = A;
-          if (2 * q + 1 < FO) o[g.ysz] = B;
-        }
+    team_sync<WAVE>();
+    if (valid) {
+      cpx<P> *oa = out + ((long)m * FO + 2 * q) * g.ysz + rr * g.xp;
+      cpx<P> *ob = oa + g.ysz;
+      for (int k = j; k < ix; k += TPX) {
+        cpx<P> A, B;
+        split_pair(tl[lpos<SW>(k)], tl[lpos<SW>((N - k) & (N - 1))], A, B);
+        st_pass<NT<P, PASS_XPASS>::st>(&oa[k], A);
+        if (2 * q + 1 < FO) st_pass<NT<P, PASS_XPASS>::st>(&ob[k], B);
       }
-      __syncthreads();
-    } else {
-      team_sync<WAVE>();
-      if (valid) {
-        cpx<P> *oa = out + ((long)m * FO + 2 * q) * g.ysz + rr * g.xp;
-        cpx<P> *ob = oa + g.ysz;
-        for (int k = j; k < ix; k += TPX) {
-          cpx<P> A, B;
-          split_pair(tl[lpos<SW>(k)], tl[lpos<SW>((N - k) & (N - 1))], A, B);
-          st_pass<NT<P, PASS_XPASS>::st>(&oa[k], A);
-          if (2 * q + 1 < FO) st_pass<NT<P, PASS_XPASS>::st>(&ob[k], B);
-        }
+    }
+  }
+}
+
+// x-pass of the 2D column-major buffers (YCol), many rows: TEAMS neighbouring rows
+// a block, whose elements k lie next to each other.  The block's threads take
+// (row, k) with the row fastest to load and store, every element once, and hand
+// them to the row teams through the LDS (rows N + 1 apart, so that the rows of one
+// k spread over the banks).  It replaces row teams that gathered their own elements
+// in 8- and 16-byte pieces and the mirrored half again (us, before -> now, FP64
+// 512^2 x 8 28.1 -> 23.6, 512^2 x 16 43.7 -> 38.0, 1024^2 x 4 63.2 -> 48.1; FP32
+// 23.7 -> 15.3, 40.8 -> 24.2, 57.8 -> 32.8).
+template <typename P, int N, int TEAMS> constexpr size_t xcol_lds() {
+  return (size_t)((N + 1) * TEAMS + N) * sizeof(cpx<P>);
+}
+template <typename P, int N, int TEAMS, int FI, int FO, class PROD>
+__global__ void __launch_bounds__(TEAMS *(N / EPT))
+k_xpass_col(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, long nrows, Grid g,
+            const cpx<P> *__restrict__ tw, PROD prod) {
+  PSG_TWIDDLES_REQUEST(P, N, EPT, TEAMS *(N / EPT));
+  constexpr int TPX = N / EPT, ix = xband<N>(), IT = (ix + TPX - 1) / TPX, RL = N + 1;
+  constexpr bool WAVE = TPX <= 64;
+  constexpr int PI = (FI + 1) / 2, PO = (FO + 1) / 2, SW = row_swizzle<EPT>();
+  // loads and stores: row r of the block, elements k0 + it TPX
+  const int r = threadIdx.x % TEAMS, k0 = threadIdx.x / TEAMS;
+  const unsigned row = (unsigned)xcd_tile().x * TEAMS + r, nrm = (unsigned)nrow_m;
+  const bool ok = row < (unsigned long)nrows;
+  const unsigned m = ok ? row / nrm : 0, y = ok ? row - m * nrm : 0;
+  cpx<P> lv[2 * PI][IT];
+#pragma unroll
+  for (int f = 0; f < 2 * PI; f++) {
+    const cpx<P> *src = in + ((long)m * FI + f) * g.ysz + y;
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+      const int k = k0 + it * TPX;
+      lv[f][it] = f < FI && ok && k < ix ? ld_pass<NT<P, PASS_XPASS>::ld>(&src[YCol::col(g, k)]) : cpx<P>{0, 0};
+      if (k == 0) lv[f][it].y = 0;
+    }
+  }
+  PSG_TWIDDLES_READY(P);
+  // transforms: row `team` of the block, thread j of its team
+  const int team = threadIdx.x / TPX, j = threadIdx.x % TPX;
+  cpx<P> *tl = lds + team * RL, *tr = lds + r * RL;
+  P phys[2 * PI][EPT];
+#pragma unroll
+  for (int p = 0; p < PI; p++) {
+    if (p) __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+      const int k = k0 + it * TPX;
+      if (k < ix) {
+        const cpx<P> a = lv[2 * p][it], b = lv[2 * p + 1][it];
+        tr[lpos<SW>(k)] = cpx<P>{a.x - b.y, a.y + b.x};
+        if (k) tr[lpos<SW>(N - k)] = cpx<P>{a.x + b.y, b.x - a.y};
+      }
+    }
+    __syncthreads();
+    cpx<P> v[EPT];
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) {
+      const int k = j + TPX * mm;
+      v[mm] = k < ix || k > N - ix ? tl[lpos<SW>(k)] : cpx<P>{0, 0};
+    }
+    team_sync<WAVE>();
+    fft_pencil<P, N, EPT, true, WAVE, SW>(v, tl, j, 1, 0, tw);
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) { phys[2 * p][mm] = v[mm].x; phys[2 * p + 1][mm] = v[mm].y; }
+  }
+  P res[2 * PO][EPT];
+#pragma unroll
+  for (int mm = 0; mm < EPT; mm++) {
+    P pin[2 * PI], pout[2 * PO];
+#pragma unroll
+    for (int f = 0; f < 2 * PI; f++) pin[f] = phys[f][mm];
+#pragma unroll
+    for (int f = 0; f < 2 * PO; f++) pout[f] = 0;
+    prod(pin, pout);
+#pragma unroll
+    for (int f = 0; f < 2 * PO; f++) res[f][mm] = pout[f];
+  }
+#pragma unroll
+  for (int q = 0; q < PO; q++) {
+    if (q) __syncthreads();
+    cpx<P> v[EPT];
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) v[mm] = cpx<P>{res[2 * q][mm], res[2 * q + 1][mm]};
+    fft_pencil<P, N, EPT, false, WAVE, SW>(v, tl, j, 1, 0, tw);
+    team_sync<WAVE>();
+#pragma unroll
+    for (int mm = 0; mm < EPT; mm++) {
+      const int k = j + TPX * mm;   // only the kept modes and their mirrors are read back
+      if (k < ix || k > N - ix) tl[lpos<SW>(k)] = v[mm];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+      const int k = k0 + it * TPX;
+      if (ok && k < ix) {
+        cpx<P> A, B;
+        split_pair(tr[lpos<SW>(k)], tr[lpos<SW>((N - k) & (N - 1))], A, B);
+        cpx<P> *o = out + ((long)m * FO + 2 * q) * g.ysz + YCol::col(g, k) + y;
+        o[0] = A;
+        if (2 * q + 1 < FO) o[g.ysz] = B;
       }
     }
   }
