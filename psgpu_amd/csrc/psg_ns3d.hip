@@ -22,7 +22,9 @@ namespace psg {
 // the working state of an FP32-bulk run).  The update is evaluated in FP64.
 // LAY: layout of st, rh and the tables (LayNKT: ik is the mode's index;
 // LayW: the working copy, indexed from the mode's wavenumbers through g)
-template <int PHASE, bool EULER, typename R = double, typename S = double, class LAY = LayNKT> struct UpdHeun {
+// FROM: the half step starts from another buffer than the one it leaves its state in
+template <int PHASE, bool EULER, typename R = double, typename S = double, class LAY = LayNKT, bool FROM = false>
+struct UpdHeun {
   cpx<S> *st;
   cpx<R> *rh;
   long ms, fs;  // member stride, field stride (same for st and rh)
@@ -31,7 +33,7 @@ template <int PHASE, bool EULER, typename R = double, typename S = double, class
   Force F;
   double dt;
   Grid g;
-  const cpx<S> *in = nullptr;  // the state the half step starts from, when it is not st itself
+  const cpx<S> *from = nullptr;
   __device__ __forceinline__ void operator()(int m, long ik_nkt, int ikx, double kx, double ky, double kz,
                                              cpx<double> (&N)[3]) const {
     PSG_CURL
@@ -42,7 +44,7 @@ template <int PHASE, bool EULER, typename R = double, typename S = double, class
       it = LayW::tab(g, ikx, iky, ikz);
     }
     cpx<S> *s = st + (long)m * ms + ik;
-    const cpx<S> *q = (in ? in : st) + (long)m * ms + ik;
+    const cpx<S> *q = (FROM ? from : st) + (long)m * ms + ik;
     cpx<R> *r = rh + (long)m * ms + ik;
     const double ll = (double)L[it];
     if constexpr (PHASE == 0) {
@@ -407,10 +409,10 @@ static int step_rec_t(Ctx *c, int umask, const cpx<double> *wn, cpx<double> *wst
   Force F{c->cfg.force, c->cfg.kf, c->cfg.ampfor};
   const long ms = 3 * g.nkt, fs = g.nkt;
   const long sb = (6 * 16 + 3 * (long)sizeof(cpx<P>)) * g.nkt;
-  UpdHeun<0, false, P> up{wstar, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g, wn};
+  UpdHeun<0, false, P, double, LayNKT, true> up{wstar, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g, wn};
   PSG_TRY(rhs3<P>(c, wn, ms, umask, up, sb, 1));
   if (!next) return 0;
-  UpdHeun<1, false, P> uc{next, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g, wstar};
+  UpdHeun<1, false, P, double, LayNKT, true> uc{next, (cpx<P> *)c->rh, ms, fs, c->nuzn, c->nu1, c->mask, F, c->cfg.dt, c->g, wstar};
   PSG_TRY(rhs3<P>(c, wstar, ms, 0, uc, sb, 1));
   return 0;
 }
