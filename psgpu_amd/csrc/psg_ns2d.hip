@@ -245,8 +245,10 @@ static int launch_xpass2(Ctx *c, const cpx<P> *in, cpx<P> *out, long nrow_m, int
       set_error("x-pass: %ld rows exceed the 32-bit row index", nrows);
       return PSG_EINVAL;
     }
-    if (nrows < 2048) {
-      // few rows: one row per block, its field pairs transformed side by side
+    // few rows: one row per block, its field pairs transformed side by side.  From 512
+    // blocks of several rows on these are faster (16 steps, three contexts at a time, one
+    // row a block and several: 1024^2 1747 and 1266 us)
+    if (nrows < (N >= 1024 ? 1024 : 2048)) {
       constexpr int NT = xsplit_teams<FI, FO>() * Row<N>::TPX;
       static_assert(NT <= 1024, "split-row x-pass block size");
       const size_t lds = xsplit_lds<P, N, FI, FO>();
