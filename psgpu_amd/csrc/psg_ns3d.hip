@@ -303,7 +303,7 @@ template <typename A, typename B, bool TO_W> static int work_copy_split(Ctx *c, 
   const Grid &g = c->g;
   const unsigned nt = (unsigned)(((g.iktx + WTX - 1) / WTX) * ((g.iktz + WTZ - 1) / WTZ));
   hipLaunchKernelGGL((k_work_split<A, B, TO_W>), dim3(nt, g.ikty, 3 * c->batch), dim3(256),
-                     sizeof(cpx<B>) * WTX * (WTZ + 1), c->stream, a, b, g, Split::of(g));
+                     sizeof(cpx<B>) * WTX * (WTZ + 1), c->stream, a, b, g, Split::of(c));
   PSG_HIP(hipGetLastError());
   return 0;
 }
@@ -345,7 +345,7 @@ __global__ void k_tables_split(const double *__restrict__ nuzn, const double *__
 int ns3d_tables_w(Ctx *c) {
   if (!c->wnuzn) return 0;
   if (c->wsplit) {
-    const Split d = Split::of(c->g);
+    const Split d = Split::of(c);
     hipLaunchKernelGGL(k_tables_split, dim3((unsigned)std::min<long>(4096, (d.nkts + 255) / 256)), dim3(256), 0, c->stream,
                        c->nuzn, c->nu1, c->mask, c->wnuzn, c->wnu1, c->wmask, c->g, d);
     PSG_HIP(hipGetLastError());
@@ -508,7 +508,7 @@ int ns3d_init(Ctx *c) {
   c->szC = (size_t)3 * g.ysz * c->batch * b;
   // the two-kernel stepper keeps F in bufB and G in bufC
   c->wsplit = split_usable(c);
-  const Split d = Split::of(g);
+  const Split d = Split::of(c);
   if (c->wsplit) {
     c->szB = std::max(c->szB, (size_t)6 * d.fs * c->batch * b);
     c->szC = std::max(c->szC, (size_t)3 * d.gs * c->batch * b);

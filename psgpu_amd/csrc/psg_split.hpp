@@ -7,7 +7,7 @@
 // part where the whole x axis is:
 //   z kernel (k_zsplit): forward y2 and z transforms of the products, Heun/CN
 //     update of the modes, velocity and inverse z and y2 transforms of the next
-//     stage's six fields, for one or two kx columns and one k1
+//     stage's six fields, for two or three kx columns and one k1
 //   xy kernel (k_xysplit): inverse y1 and x transforms, product, forward x and
 //     y1 transforms, for one (z, y2): 16 rows
 // Between them move F (six fields, [f][kx group][k1][y2][z][kb]) and G (three
@@ -23,21 +23,30 @@ namespace psg {
 
 constexpr int SPLIT_RB = 16;   // rows of the xy kernel, points of its y transform
 
-// kx columns per z-kernel block: G and F move in pieces of kb points
-__host__ __device__ constexpr int split_kb(int nz, int ra) { return nz * ra >= 1024 ? 3 : 2; }
+// kx columns per z-kernel block: G and F move in pieces of kb points.  Two make
+// pieces of 32 bytes in FP64; in FP32 they make 16, and from 1024 (z, y2) points a
+// column on three are taken: fewer pieces, for more threads a block (864 instead of
+// 576) and fewer blocks.  In FP64 the larger blocks cost more than they give.  One
+// step in us, one context / three at a time, two columns and three:
+//   FP64 32x128x128 84.8 / 43.7, 117 / 50.8; 64x128x128 96.9 / 71.8, 127 / 85.9
+//   FP32 128^3 130 / 95.1, 105 / 89.1; 64x128x128 x 2 131 / 97.1, 105 / 92.7;
+//        64x128x128 84.5 / 52.8, 91.1 / 46.6; 32x128x128 74.1 / 33.4, 84.7 / 35.2
+__host__ __device__ constexpr int split_kb(bool fp32, int nz, int ra) { return fp32 && nz * ra >= 1024 ? 3 : 2; }
 
 // sizes and pitches of the split buffers and of the working layout
 struct Split {
-  int ra, kb, ng;    // y2 count; kx columns of a z-kernel block (1 or 2); groups of kb columns
-  int pa;            // points of one (group, k1) chunk of F: ra nz kb, padded to an odd number of lines
+  int ra, kb, ng;    // y2 count; kx columns of a z-kernel block (split_kb); groups of kb columns
+  int pa;            // points of one (group, k1) chunk of F: ra nz kb, and 8 so that in FP64 chunks
+                     // start an odd number of 128-byte lines apart (in FP32 of half lines)
   int xq, zp;        // kx pitch of a G row; points of one z plane of G (likewise padded)
   int kzp;           // kz pitch of the working state [ikx][iky][f][kz], kz = 0..KTZ, -KTZ..-1
   long fs, gs;       // points per field of F and G
   long nkts;         // working modes per field
-  __host__ __device__ static Split of(const Grid &g) {
+  static Split of(const Ctx *c) {
+    const Grid &g = c->g;
     Split s;
     s.ra = g.ny / SPLIT_RB;
-    s.kb = split_kb(g.nz, s.ra);
+    s.kb = split_kb(c->cfg.precision == PSG_FP32BULK, g.nz, s.ra);
     s.ng = (g.iktx + s.kb - 1) / s.kb;
     s.pa = s.ra * g.nz * s.kb + 8;
     s.xq = (g.iktx + 7) / 8 * 8;
@@ -65,12 +74,12 @@ struct SplitUpd {
   Force F;
 };
 
-template <int NZ, int RA> struct ZShape {
+template <typename P, int NZ, int RA> struct ZShape {
   static constexpr int TP = NZ / EPT;
   static constexpr int NC = 2 * RA / 3 + 1;      // columns p = k1 + 16 k2 inside the 2/3 band, at most
-  static constexpr int KB = split_kb(NZ, RA), COLS = KB * NC;
+  static constexpr int KB = split_kb(sizeof(P) == 4, NZ, RA), COLS = KB * NC;
   static constexpr int NT = 3 * COLS * TP;
-  template <typename P> static constexpr size_t lds() { return (size_t)(NZ + 3 * COLS * NZ) * sizeof(cpx<P>); }
+  static constexpr size_t lds() { return (size_t)(NZ + 3 * COLS * NZ) * sizeof(cpx<P>); }
 };
 
 // One block: kb columns of kx, one k1, all k2 and kz, three fields side by side
@@ -80,11 +89,11 @@ template <int NZ, int RA> struct ZShape {
 // their new values itself, from its own transforms (the products are real, so
 // N(-k) = conj N(k)), and must find their old values whole.
 template <typename P, int NZ, int RA>
-__global__ void __launch_bounds__((ZShape<NZ, RA>::NT)) PSG_WAVES_PER_EU((sizeof(P) == 4 ? 4 : 3))
+__global__ void __launch_bounds__((ZShape<P, NZ, RA>::NT)) PSG_WAVES_PER_EU((sizeof(P) == 4 ? 4 : 3))
 k_zsplit(const cpx<P> *__restrict__ G, cpx<P> *__restrict__ F, const cpx<P> *__restrict__ st, cpx<P> *__restrict__ sn,
          cpx<P> *__restrict__ rh, const double *__restrict__ nuzn, const double *__restrict__ nu1,
          const int8_t *__restrict__ L, Grid g, Split d, const cpx<P> *__restrict__ tw, SplitUpd u) {
-  using Z = ZShape<NZ, RA>;
+  using Z = ZShape<P, NZ, RA>;
   constexpr int E = EPT, TP = Z::TP, NT = Z::NT, KB = Z::KB, COLS = Z::COLS;
   constexpr int SW = row_swizzle<E>();
   PSG_TWIDDLES_REQUEST(P, NZ, E, NT);
@@ -470,15 +479,21 @@ inline bool split_len(int n) { return n == 32 || n == 64 || n == 128; }
 // of the 256 MB last-level cache, and the default kernel shapes (the others are
 // those of the five pencil passes).  What the split saves is launches and their
 // latency; its pieces of kb points cost more than the pencil passes' 128-byte
-// ones once F and G come from HBM.  One step, FP64, three contexts at a time,
-// pencil passes -> two kernels: 32^3 25.6 -> 14.5 us, 64^3 37.6 -> 22.7, 64^3 x 4
-// (52 MB) 87.0 -> 54.4, 128x128x64 (51 MB) 86.2 -> 80.8, but 128^3 (101 MB)
-// 167 -> 190 and, in FP32, 128x128x64 x 4 (101 MB) 189 -> 208; 256^3 1320 -> 1920.
+// ones once F and G come from HBM.  One step in us, pencil passes -> two kernels:
+//   one context: FP64 32x128x128 108 -> 84, 64x128x128 132 -> 98, 128x128x64 129 -> 113;
+//     FP32 64x128x128 x 2 148 -> 105, 128^3 138 -> 105
+//   three at a time: FP64 32^3 25.6 -> 14.5, 64^3 37.6 -> 22.7, 64^3 x 4 (52 MB)
+//     87.0 -> 54.4, 128x128x64 (51 MB) 86.2 -> 80.8; FP32 128^3 98 -> 88
+// Beyond the line it depends on what else runs: at about 100 MB a context that has
+// the cache to itself still gains (FP64 128^3 206 -> 183, FP32 128x128x64 x 4
+// 242 -> 229), three of them lose (167 -> 177, 196 -> 214) or, with short rows, not
+// (64^3 x 8 188 -> 137).  A context cannot know its neighbours, and no grid within
+// the line is slower either way, so the line stands where both agree.
 inline bool split_usable(const Ctx *c) {
   if (c->g.dim != 3 || c->cfg.flavour == PSG_BOUS3D || !split_len(c->g.nx) || !split_len(c->g.ny) || !split_len(c->g.nz))
     return false;
   if (c->xvar || c->zvar || c->slvar) return false;
-  const Split d = Split::of(c->g);
+  const Split d = Split::of(c);
   const size_t b = c->cfg.precision == PSG_FP32BULK ? 8 : 16;
   return (6 * d.fs + 3 * d.gs) * (size_t)c->batch * b <= (size_t)64 << 20;
 }
@@ -487,7 +502,7 @@ inline bool split_usable(const Ctx *c) {
 // and writes the second, phase 1 the other way round
 template <typename P> static int launch_zsplit(Ctx *c, cpx<P> *st, SplitUpd u) {
   const Grid &g = c->g;
-  const Split d = Split::of(g);
+  const Split d = Split::of(c);
   cpx<P> *st2 = st + 3 * d.nkts * c->batch;
   auto go = [&](auto k, int nt, size_t lds) -> int {
     PSG_HIP(lds_attr(k, lds));
@@ -500,7 +515,7 @@ template <typename P> static int launch_zsplit(Ctx *c, cpx<P> *st, SplitUpd u) {
   auto len = [&](auto ra) -> int {
     constexpr int RA = decltype(ra)::value;
     switch (g.nz) {
-#define PSG_ZS(NZ) case NZ: return go(k_zsplit<P, NZ, RA>, ZShape<NZ, RA>::NT, ZShape<NZ, RA>::template lds<P>());
+#define PSG_ZS(NZ) case NZ: return go(k_zsplit<P, NZ, RA>, ZShape<P, NZ, RA>::NT, ZShape<P, NZ, RA>::lds());
       PSG_ZS(32) PSG_ZS(64) PSG_ZS(128)
 #undef PSG_ZS
     }
@@ -518,7 +533,7 @@ template <typename P> static int launch_zsplit(Ctx *c, cpx<P> *st, SplitUpd u) {
 
 template <typename P> static int launch_xysplit(Ctx *c) {
   const Grid &g = c->g;
-  const Split d = Split::of(g);
+  const Split d = Split::of(c);
   const int units = g.nz * d.ra * c->batch;
   auto go = [&](auto k, int nt, size_t lds) -> int {
     PSG_HIP(lds_attr(k, lds));
