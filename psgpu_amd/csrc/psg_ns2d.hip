@@ -245,9 +245,22 @@ static int launch_xpass2(Ctx *c, const cpx<P> *in, cpx<P> *out, long nrow_m, int
       set_error("x-pass: %ld rows exceed the 32-bit row index", nrows);
       return PSG_EINVAL;
     }
-    // few rows: one row per block, its field pairs transformed side by side.  From 512
-    // blocks of several rows on these are faster (16 steps, three contexts at a time, one
-    // row a block and several: 1024^2 1747 and 1266 us)
+    // few rows: one row per block, its field pairs transformed side by side.  Several rows
+    // a block gather whole pieces of lines, but are fewer blocks with a longer chain each:
+    // they win from 2048 rows on at every length (from 1024 rows on also at 1024 points)
+    // and lose on the few rows of a single small grid.  Us, one row a block and several:
+    //   step, FP64, one context (three at a time):
+    //      64 points   512 rows 40.4, 40.8 (15.8, 15.9)   2048 rows 47.4, 42.2 (21.1, 18.1)
+    //     128 points   512 rows 44.2, 49.1 (19.1, 20.7)   2048 rows 59.1, 51.1 (29.6, 23.3)
+    //     256 points  1024 rows 64.8, 62.9 (30.3, 26.7)   2048 rows 78.4, 62.5 (47.7, 34.9)
+    //     512 points   512 rows 68.9, 65.6 (31.8, 28.1)   1024 rows 97.6, 83.8 (50.7, 36.4)
+    //    1024 points   256 rows 75.9, 77.4 (40.6, 32.6)   1024 rows  190,  154 ( 109, 80.2)
+    //   the same in FP32: 16 points 2048 rows 44.6, 41.7 (15.9, 16.1), 64 points 2048 rows
+    //     40.7, 37.6 (17.1, 15.5), 1024 points 256 rows 61.6, 68.2 (28.1, 28.8), 1024 rows
+    //     149, 112 (84.9, 54.0)
+    //   tangent of 20 steps (6 fields in, 4 out), one context, FP64 and FP32: 64 points 2048
+    //     rows 1288, 1293 and 1077, 1098; 128 points 2048 rows 1747, 1661 and 1398, 1288;
+    //     512^2 2364, 2295 and 1875, 1900; 1024^2 8656, 6033 and 5849, 4137
     if (nrows < (N >= 1024 ? 1024 : 2048)) {
       constexpr int NT = xsplit_teams<FI, FO>() * Row<N>::TPX;
       static_assert(NT <= 1024, "split-row x-pass block size");
@@ -257,10 +270,12 @@ static int launch_xpass2(Ctx *c, const cpx<P> *in, cpx<P> *out, long nrow_m, int
       hipLaunchKernelGGL(k, dim3((unsigned)nrows), dim3(NT), lds, c->stream, in, out, nrow_m, nrows, g,
                          twp<P>(c, 0), prod);
     } else {
-      // rows per block: pieces of 64 bytes from 512 points on, lines below.  Twice the rows
-      // leaves one or two blocks a CU, whose barriers then stand alone (FP64 us, this and
-      // twice: 512^2 x 8 23.6, 27.3; 1024^2 x 4 48.1, 64.3); half of them in FP32 gathers
-      // 32 bytes (FP32 512^2 x 8 15.3, 15.8; 1024^2 x 2 20.3, 21.7)
+      // rows per block: 256 threads, 512 for the long rows in FP32 (128 rows at 16 points, 4 at
+      // 512 and 2 at 1024 in FP64, 8 and 4 in FP32).  They gather pieces of 128 bytes and more
+      // in FP64 up to 256 points, of 64 at 512 and 32 at 1024.  Twice the rows leaves one or two
+      // blocks a CU, whose barriers then stand alone (FP64 us, this and twice: 512^2 x 8 23.6,
+      // 27.3; 1024^2 x 4 48.1, 64.3); half of them halves the pieces (FP32 512^2 x 8 15.3,
+      // 15.8; 1024^2 x 2 20.3, 21.7)
       constexpr int TE = Row<N>::TEAMS * (sizeof(P) == 4 && N >= 512 ? 2 : 1);
       constexpr size_t lds = xcol_lds<P, N, TE>();
       static_assert(TE * Row<N>::TPX <= 1024 && lds <= 160 * 1024, "column x-pass block size");
