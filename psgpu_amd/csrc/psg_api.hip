@@ -270,7 +270,7 @@ static void free_ctx(Ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (auto &e : c->graph_exec)
     if (e) { (void)hipGraphExecDestroy(e); e = nullptr; }
-  void *ptrs[] = {c->state, c->rh, c->stage, c->tmp, c->st32, c->stw, c->wnuzn, c->wnu1, c->wmask, c->nuzn, c->nu1, c->nu, c->mask, c->tl_state, c->tl_stage,
+  void *ptrs[] = {c->state, c->rh, c->stage, c->tmp, c->st32, c->stw, c->wnuzn, c->wnu1, c->wmask, c->nuzn, c->nu1, c->nu, c->mask, c->tl_state,
                   c->tl_rh, c->tl_bufA, c->tl_bufB, c->tl_bufC, c->bufA, c->bufB, c->bufC,
                   c->tw64[0], c->tw64[1], c->tw64[2], c->tw32[0], c->tw32[1], c->tw32[2], c->dred, c->io, c->dtm,
                   c->rec, c->rec_cnt, c->adj};
@@ -374,8 +374,7 @@ static int run_steps_in(Ctx *c, int kind, int nsteps) {
 }
 
 void tl_free(Ctx *c) {
-  for (void **p : {(void **)&c->tl_state, (void **)&c->tl_stage, (void **)&c->tl_rh, &c->tl_bufA, &c->tl_bufB,
-                   &c->tl_bufC}) {
+  for (void **p : {(void **)&c->tl_state, (void **)&c->tl_rh, &c->tl_bufA, &c->tl_bufB, &c->tl_bufC}) {
     if (*p) (void)hipFree(*p);
     *p = nullptr;
   }
@@ -385,14 +384,12 @@ void tl_free(Ctx *c) {
 // the pointers are null again, so a later call retries instead of running
 // kernels on a partial set.
 int tl_alloc(Ctx *c) {
-  if (c->tl_state && c->tl_stage && c->tl_rh && c->tl_bufB && c->tl_bufC && (c->g.dim == 2 || c->tl_bufA))
-    return 0;
+  if (c->tl_state && c->tl_rh && c->tl_bufB && c->tl_bufC && (c->g.dim == 2 || c->tl_bufA)) return 0;
   tl_free(c);
   const Grid &g = c->g;
   const size_t sb = sizeof(cpx<double>) * c->nf * g.nkt * c->batch;
   const size_t b = c->cfg.precision == PSG_FP32BULK ? sizeof(cpx<float>) : sizeof(cpx<double>);
-  bool ok = hipMalloc(&c->tl_state, sb) == hipSuccess && hipMalloc(&c->tl_stage, sb) == hipSuccess &&
-            hipMalloc(&c->tl_rh, 3 * sb) == hipSuccess;
+  bool ok = hipMalloc(&c->tl_state, sb) == hipSuccess && hipMalloc(&c->tl_rh, sb) == hipSuccess;
   if (ok && g.dim == 2)
     ok = hipMalloc(&c->tl_bufB, 6 * g.ysz * c->batch * b) == hipSuccess &&
          hipMalloc(&c->tl_bufC, 4 * g.ysz * c->batch * b) == hipSuccess;
@@ -401,8 +398,7 @@ int tl_alloc(Ctx *c) {
          hipMalloc(&c->tl_bufB, 12 * g.ysz * c->batch * b) == hipSuccess &&
          hipMalloc(&c->tl_bufC, 6 * g.ysz * c->batch * b) == hipSuccess;
   ok = ok && hipMemsetAsync(c->tl_state, 0, sb, c->stream) == hipSuccess &&
-       hipMemsetAsync(c->tl_stage, 0, sb, c->stream) == hipSuccess &&
-       hipMemsetAsync(c->tl_rh, 0, 3 * sb, c->stream) == hipSuccess;
+       hipMemsetAsync(c->tl_rh, 0, sb, c->stream) == hipSuccess;
   if (!ok) {
     (void)hipGetLastError();
     tl_free(c);

@@ -53,8 +53,8 @@ struct Ctx {
   int cus = 256;   // compute units of the device
   // state and scheme arrays (FP64 complex), member-major [batch][nf][nkt]
   cpx<double> *state = nullptr;
-  cpx<double> *rh = nullptr;        // Heun: RH store; RK4: stage arrays
-  cpx<double> *stage = nullptr;     // RK4: Z0 stage input / generic scratch
+  cpx<double> *rh = nullptr;        // Heun: RH store; 2D RK4: running sum of the increments; Boussinesq: the increments
+  cpx<double> *stage = nullptr;     // Boussinesq: stage input Z0
   cpx<double> *tmp = nullptr;       // scratch state-sized buffer
   // 3D Navier-Stokes/Euler: working copy of the state during a run, in the
   // layout LayW of the five pencil passes or Split::at of the two-kernel
@@ -81,9 +81,9 @@ struct Ctx {
   double *dtm = nullptr;
   bool dtm_on = false;
   // tangent-linear companion state (allocated on first use): perturbation,
-  // its stage input and stage increments, and pass buffers sized for the
-  // combined base + perturbation transforms
-  cpx<double> *tl_state = nullptr, *tl_stage = nullptr, *tl_rh = nullptr;
+  // what rh holds of it, and pass buffers sized for the combined base +
+  // perturbation transforms
+  cpx<double> *tl_state = nullptr, *tl_rh = nullptr;
   bool tl_fp32 = false;             // tangent-linear passes in FP32-bulk in an FP64 context
   void *tl_bufA = nullptr, *tl_bufB = nullptr, *tl_bufC = nullptr;
   // adjoint sweep: recorded states and work fields, kept up to 1 GiB (a gradient
