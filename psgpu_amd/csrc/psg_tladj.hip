@@ -284,8 +284,8 @@ struct Sweep {
   int n, K, nseg;
   long n3;
   bool opened = false;
-  // nothing of the call is in flight when it returns, also on an error; a large
-  // workspace is given back
+  // nothing of the call is in flight when it returns, also on an error; a workspace
+  // above 1 GiB is given back, a smaller one stays for the next sweep
   ~Sweep() {
     if (!opened) return;
     (void)hipStreamSynchronize(c->stream);
