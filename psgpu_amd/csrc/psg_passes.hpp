@@ -607,9 +607,12 @@ k_xpass(const cpx<P> *__restrict__ in, cpx<P> *__restrict__ out, long nrow_m, lo
   constexpr int ix = xband<N>();
   const long ro = YTile<P>::row(g, (int)y, (int)z);
   auto rowp = [&](int f) { return in + ((long)m * FI + f) * g.ysz + ro; };
-  // nine front-loaded fields leave no registers for the twiddles' trip (the
-  // FP32 256-point Boussinesq pass ran 0.5% slower with it)
-  constexpr bool TWFIRST = FI > 6;
+  // the twiddles go ahead of the data where no registers are left for their trip: nine
+  // front-loaded fields (the FP32 256-point Boussinesq pass ran 0.5% slower with it), and
+  // the register caps that spill already (us, six fields, twiddles beside the data and
+  // ahead: five FP64 waves 256^3 490 and 454, 512x128^2 278 and 264; four at 128^3 41.6
+  // and 40.2, six FP32 waves there 26.4 and 25.6; the other caps gain like the rest)
+  constexpr bool TWFIRST = FI > 6 || (WPE > 0 && (N <= 128 || (sizeof(P) == 8 && WPE >= 5)));
   if constexpr (TWFIRST) PSG_TWIDDLES_READY(P);
   cpx<P> vin[NV][E];
   if constexpr (FRONT) {
