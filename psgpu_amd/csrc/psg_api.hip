@@ -303,13 +303,13 @@ int timederiv_dev(Ctx *c, const cpx<double> *in, cpx<double> *out) {
   return 0;
 }
 
-static int run_eager(Ctx *c, int kind, int n, bool first) {
+static int run_eager(Ctx *c, int kind, int n, bool first, bool last) {
   if (n <= 0) return 0;
-  if (kind == 1) return c->g.dim == 2 ? ns2d_tl_run(c, n, first) : ns3d_tl_run(c, n, first);
-  if (kind == 2) return ns2d_rec_run(c, n, first);
-  if (kind == 3) return ns2d_tlrec_run(c, n, first);
-  if (c->g.dim == 2) return ns2d_run(c, n, first);
-  return c->cfg.flavour == PSG_BOUS3D ? bous_run(c, n, first) : ns3d_run(c, n, first);
+  if (kind == 1) return c->g.dim == 2 ? ns2d_tl_run(c, n, first, last) : ns3d_tl_run(c, n, first);
+  if (kind == 2) return ns2d_rec_run(c, n, first, last);
+  if (kind == 3) return ns2d_tlrec_run(c, n, first, last);
+  if (c->g.dim == 2) return ns2d_run(c, n, first, last);
+  return c->cfg.flavour == PSG_BOUS3D ? bous_run(c, n, first) : ns3d_run(c, n, first, last);
 }
 
 // Capture graph_steps steps (all launches, no memsets or host work) into an
@@ -323,7 +323,7 @@ static int build_graph(Ctx *c, int kind) {
   }
   hipGraph_t g = nullptr;
   if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return -1;
-  const int r = run_eager(c, kind, c->graph_steps, false);
+  const int r = run_eager(c, kind, c->graph_steps, false, false);
   const hipError_t e = hipStreamEndCapture(c->stream, &g);
   if (r || e != hipSuccess || !g) {
     if (g) (void)hipGraphDestroy(g);
@@ -359,18 +359,18 @@ int run_steps(Ctx *c, int kind, int nsteps) {
 
 static int run_steps_in(Ctx *c, int kind, int nsteps) {
   const int G = c->graph_steps;
-  if (G <= 0 || c->prof || c->graph_failed || nsteps < G + 1) return run_eager(c, kind, nsteps, true);
+  if (G <= 0 || c->prof || c->graph_failed || nsteps < G + 1) return run_eager(c, kind, nsteps, true, true);
   // the first step of a call is eager: it may mask the velocity / copy the stage input
-  if (int r = run_eager(c, kind, 1, true)) return r;
+  if (int r = run_eager(c, kind, 1, true, false)) return r;
   int left = nsteps - 1;
   if (c->graph_built[kind] != c->graph_gen || !c->graph_exec[kind]) {
     if (build_graph(c, kind)) {
       c->graph_failed = true;
-      return run_eager(c, kind, left, false);
+      return run_eager(c, kind, left, false, true);
     }
   }
   for (; left >= G; left -= G) PSG_HIP(hipGraphLaunch(c->graph_exec[kind], c->stream));
-  return run_eager(c, kind, left, false);
+  return run_eager(c, kind, left, false, true);
 }
 
 void tl_free(Ctx *c) {

@@ -164,7 +164,9 @@ void prof_end(Ctx *c);
 
 // per-flavour drivers
 int ns3d_init(Ctx *c);
-int ns3d_run(Ctx *c, int nsteps, bool first);
+// first, last: the first and the last steps of a run (the steppers that make the next
+// stage's fields with an update make none at the end)
+int ns3d_run(Ctx *c, int nsteps, bool first, bool last);
 int ns3d_work_begin(Ctx *c);
 int ns3d_work_end(Ctx *c);
 int ns3d_tables_w(Ctx *c);
@@ -174,7 +176,7 @@ int ns3d_physical(Ctx *c, int member, double *out_dev);
 int ns3d_physical_state(Ctx *c, const cpx<double> *st, double *out_dev);
 int set_member_dt(Ctx *c, const double *host);
 int ns2d_init(Ctx *c);
-int ns2d_run(Ctx *c, int nsteps, bool first);
+int ns2d_run(Ctx *c, int nsteps, bool first, bool last);
 int ns2d_nonlin(Ctx *c, int member, const cpx<double> *in_dev, cpx<double> *out_dev);
 int ns2d_physical(Ctx *c, int member, double *out_dev);
 int diag_member(Ctx *c, int member, double *e, double *z, double *spec);
@@ -185,10 +187,10 @@ int bous_physical(Ctx *c, int member, double *out_dev);
 // physical fields (xi, eta, zeta, u, v, w, rho) of a Boussinesq state held anywhere in device memory
 int bous_physical_state(Ctx *c, const cpx<double> *st, double *out_dev);
 int timederiv_dev(Ctx *c, const cpx<double> *in, cpx<double> *out);
-int ns2d_tl_run(Ctx *c, int nsteps, bool first);
+int ns2d_tl_run(Ctx *c, int nsteps, bool first, bool last);
 int ns3d_tl_run(Ctx *c, int nsteps, bool first);
-int ns2d_rec_run(Ctx *c, int nsteps, bool first);
-int ns2d_tlrec_run(Ctx *c, int nsteps, bool first);
+int ns2d_rec_run(Ctx *c, int nsteps, bool first, bool last);
+int ns2d_tlrec_run(Ctx *c, int nsteps, bool first, bool last);
 // nsteps of the plain (kind 0), tangent-linear (kind 1), base-recording (kind 2)
 // or recorded tangent-linear (kind 3) stepper: an eager first step, then
 // replays of a captured graph of graph_steps steps

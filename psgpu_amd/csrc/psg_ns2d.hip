@@ -306,8 +306,17 @@ template <int S> static Upd2D<S> pert2(const Ctx *c, int *cnt = nullptr) {
 }
 static Load2D load2(const Ctx *c, const cpx<double> *z) { return Load2D{z, c->g.nkt, c->mask}; }
 
+// the column pass that ends a stage; a run's last stage (end) only updates the state
+template <typename P, int S, int NG = 1>
+static int col2_stage(Ctx *c, const cpx<P> *in, cpx<P> *out, int nm, Upd2D<S> u0, Upd2D<S> u1, bool end) {
+  if constexpr (S == 3) {
+    if (end) return launch_col2<P, true, false, Upd2D<S>, NG>(c, in, out, nm, u0, u1);
+  }
+  return launch_col2<P, true, true, Upd2D<S>, NG>(c, in, out, nm, u0, u1);
+}
+
 // one stage from the y-space fields in B, which it leaves ready for the next
-template <typename P, class UPD> static int stage2(Ctx *c, UPD upd, int nm) {
+template <typename P, int S> static int stage2(Ctx *c, Upd2D<S> upd, int nm, bool end) {
   const Grid &g = c->g;
   cpx<P> *B = (cpx<P> *)c->bufB, *Cb = (cpx<P> *)c->bufC;
   const long Y = (long)g.iktx * g.ny;
@@ -316,25 +325,28 @@ template <typename P, class UPD> static int stage2(Ctx *c, UPD upd, int nm) {
   PSG_TRY2((launch_xpass2<P, 3, 2>(c, B, Cb, g.ny, nm, Prod2D<P>{})));
   prof_end(c);
   prof_begin(c, "ycol2_update", (long)(5 * Y * b + 3 * g.nkt * 16) * nm);
-  PSG_TRY2((launch_col2<P, true, true>(c, Cb, B, nm, upd)));
+  PSG_TRY2((col2_stage<P, S>(c, Cb, B, nm, upd, upd, end)));
   prof_end(c);
   return 0;
 }
 
-template <typename P> static int run2_t(Ctx *c, int nsteps, bool first) {
-  // a run starts from the masked state; every later stage finds its fields in B
+// first, last: the first and the last steps of a run.  It starts from the masked state,
+// every later stage finds its fields in B, and its last stage makes none (runs of one
+// step, 1024^2 x 4 in three contexts: 389 us with the unused transforms, 367 without)
+template <typename P> static int run2_t(Ctx *c, int nsteps, bool first, bool last) {
   if (first) PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, (cpx<P> *)c->bufB, c->batch, load2(c, c->state))));
   for (int nt = 0; nt < nsteps; nt++) {
-    PSG_TRY2(stage2<P>(c, upd2<0>(c), c->batch));
-    PSG_TRY2(stage2<P>(c, upd2<1>(c), c->batch));
-    PSG_TRY2(stage2<P>(c, upd2<2>(c), c->batch));
-    PSG_TRY2(stage2<P>(c, upd2<3>(c), c->batch));
+    const bool end = last && nt == nsteps - 1;
+    PSG_TRY2((stage2<P>(c, upd2<0>(c), c->batch, end)));
+    PSG_TRY2((stage2<P>(c, upd2<1>(c), c->batch, end)));
+    PSG_TRY2((stage2<P>(c, upd2<2>(c), c->batch, end)));
+    PSG_TRY2((stage2<P>(c, upd2<3>(c), c->batch, end)));
   }
   return 0;
 }
 
-int ns2d_run(Ctx *c, int nsteps, bool first) {
-  return c->cfg.precision == PSG_FP32BULK ? run2_t<float>(c, nsteps, first) : run2_t<double>(c, nsteps, first);
+int ns2d_run(Ctx *c, int nsteps, bool first, bool last) {
+  return c->cfg.precision == PSG_FP32BULK ? run2_t<float>(c, nsteps, first, last) : run2_t<double>(c, nsteps, first, last);
 }
 
 template <typename P> static int nonlin2_t(Ctx *c, const cpx<double> *in, cpx<double> *out) {
@@ -407,30 +419,31 @@ int ns2d_physical(Ctx *c, int member, double *out_dev) {
 // dN = -i(kx FFT(du w + u dw) + ky FFT(dv w + v dw)) (no forcing) with the
 // same damping factors and masks as the base update.  The x-pass mixes them;
 // the column pass takes them as two independent groups.
-template <typename P, int S> static int stage2_tl(Ctx *c) {
+template <typename P, int S> static int stage2_tl(Ctx *c, bool end) {
   cpx<P> *B = (cpx<P> *)c->tl_bufB, *Cb = (cpx<P> *)c->tl_bufC;
   Upd2D<S> base = upd2<S>(c);
   base.dtm = nullptr;
   PSG_TRY2((launch_xpass2<P, 6, 4>(c, B, Cb, c->g.ny, c->batch, Prod2DTL<P>{})));
-  return launch_col2<P, true, true, Upd2D<S>, 2>(c, Cb, B, c->batch, base, pert2<S>(c));
+  return col2_stage<P, S, 2>(c, Cb, B, c->batch, base, pert2<S>(c), end);
 }
 
-template <typename P> static int run2tl_t(Ctx *c, int nsteps, bool first) {
+template <typename P> static int run2tl_t(Ctx *c, int nsteps, bool first, bool last) {
   if (first)
     PSG_TRY2((launch_col2<P, false, true, Load2D, 2>(c, nullptr, (cpx<P> *)c->tl_bufB, c->batch, load2(c, c->state),
                                                      load2(c, c->tl_state))));
   for (int nt = 0; nt < nsteps; nt++) {
-    PSG_TRY2((stage2_tl<P, 0>(c)));
-    PSG_TRY2((stage2_tl<P, 1>(c)));
-    PSG_TRY2((stage2_tl<P, 2>(c)));
-    PSG_TRY2((stage2_tl<P, 3>(c)));
+    const bool end = last && nt == nsteps - 1;
+    PSG_TRY2((stage2_tl<P, 0>(c, end)));
+    PSG_TRY2((stage2_tl<P, 1>(c, end)));
+    PSG_TRY2((stage2_tl<P, 2>(c, end)));
+    PSG_TRY2((stage2_tl<P, 3>(c, end)));
   }
   return 0;
 }
 
-int ns2d_tl_run(Ctx *c, int nsteps, bool first) {
-  return (c->cfg.precision == PSG_FP32BULK || c->tl_fp32) ? run2tl_t<float>(c, nsteps, first)
-                                                          : run2tl_t<double>(c, nsteps, first);
+int ns2d_tl_run(Ctx *c, int nsteps, bool first, bool last) {
+  return (c->cfg.precision == PSG_FP32BULK || c->tl_fp32) ? run2tl_t<float>(c, nsteps, first, last)
+                                                          : run2tl_t<double>(c, nsteps, first, last);
 }
 
 // ------------------------------------------------------------------ recorded base
@@ -533,7 +546,7 @@ static int launch_xpass2_split(Ctx *c, const cpx<P> *in, cpx<P> *out, PROD prod)
   return 0;
 }
 
-template <typename P, typename RP> static int run2rec_t(Ctx *c, int nsteps, bool first) {
+template <typename P, typename RP> static int run2rec_t(Ctx *c, int nsteps, bool first, bool last) {
   const Grid &g = c->g;
   if (c->batch != 1 || !c->rec || !c->rec_cnt) {
     set_error("recorded base: one member and an allocated record only");
@@ -542,11 +555,13 @@ template <typename P, typename RP> static int run2rec_t(Ctx *c, int nsteps, bool
   cpx<P> *B = (cpx<P> *)c->bufB, *Cb = (cpx<P> *)c->bufC;
   if (first) PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, B, 1, load2(c, c->state))));
   for (int nt = 0; nt < nsteps; nt++) {
+    const bool end = last && nt == nsteps - 1;
 #define PSG_REC_STAGE(S)                                                           \
     {                                                                              \
       Prod2DRec<P, RP> pr{(RP *)c->rec, c->rec_cnt, S, c->rec_slots, g.nx, g.ny};  \
       PSG_TRY2((launch_xpass2_split<P, 3, 2>(c, B, Cb, pr)));                      \
-      PSG_TRY2((launch_col2<P, true, true>(c, Cb, B, 1, upd2<S>(c, c->rec_cnt)))); \
+      const Upd2D<S> u = upd2<S>(c, c->rec_cnt);                                   \
+      PSG_TRY2((col2_stage<P, S>(c, Cb, B, 1, u, u, end)));                        \
     }
     PSG_REC_STAGE(0) PSG_REC_STAGE(1) PSG_REC_STAGE(2) PSG_REC_STAGE(3)
 #undef PSG_REC_STAGE
@@ -554,7 +569,7 @@ template <typename P, typename RP> static int run2rec_t(Ctx *c, int nsteps, bool
   return 0;
 }
 
-template <typename P> static int run2tlrec_t(Ctx *c, int nsteps, bool first) {
+template <typename P> static int run2tlrec_t(Ctx *c, int nsteps, bool first, bool last) {
   const Grid &g = c->g;
   if (c->batch != 1 || !c->rec || !c->rec_cnt || c->rec_p != (int)sizeof(P)) {
     set_error("recorded tangent linear: one member and a record of the pass precision only");
@@ -563,11 +578,13 @@ template <typename P> static int run2tlrec_t(Ctx *c, int nsteps, bool first) {
   cpx<P> *B = (cpx<P> *)c->tl_bufB, *Cb = (cpx<P> *)c->tl_bufC;
   if (first) PSG_TRY2((launch_col2<P, false, true>(c, (const cpx<P> *)nullptr, B, 1, load2(c, c->tl_state))));
   for (int nt = 0; nt < nsteps; nt++) {
+    const bool end = last && nt == nsteps - 1;
 #define PSG_TLR_STAGE(S)                                                                \
     {                                                                                   \
       Prod2DTLRec<P, P> pr{(const P *)c->rec, c->rec_cnt, S, c->rec_slots, g.nx, g.ny}; \
       PSG_TRY2((launch_xpass2_split<P, 3, 2>(c, B, Cb, pr)));                           \
-      PSG_TRY2((launch_col2<P, true, true>(c, Cb, B, 1, pert2<S>(c, c->rec_cnt))));     \
+      const Upd2D<S> u = pert2<S>(c, c->rec_cnt);                                       \
+      PSG_TRY2((col2_stage<P, S>(c, Cb, B, 1, u, u, end)));                             \
     }
     PSG_TLR_STAGE(0) PSG_TLR_STAGE(1) PSG_TLR_STAGE(2) PSG_TLR_STAGE(3)
 #undef PSG_TLR_STAGE
@@ -575,16 +592,16 @@ template <typename P> static int run2tlrec_t(Ctx *c, int nsteps, bool first) {
   return 0;
 }
 
-int ns2d_rec_run(Ctx *c, int nsteps, bool first) {
+int ns2d_rec_run(Ctx *c, int nsteps, bool first, bool last) {
   if (c->cfg.precision == PSG_FP32BULK) {
     if (c->rec_p != 4) { set_error("recorded base: an FP32-bulk context records FP32"); return PSG_EINVAL; }
-    return run2rec_t<float, float>(c, nsteps, first);
+    return run2rec_t<float, float>(c, nsteps, first, last);
   }
-  return c->rec_p == 4 ? run2rec_t<double, float>(c, nsteps, first) : run2rec_t<double, double>(c, nsteps, first);
+  return c->rec_p == 4 ? run2rec_t<double, float>(c, nsteps, first, last) : run2rec_t<double, double>(c, nsteps, first, last);
 }
 
-int ns2d_tlrec_run(Ctx *c, int nsteps, bool first) {
-  return c->rec_p == 4 ? run2tlrec_t<float>(c, nsteps, first) : run2tlrec_t<double>(c, nsteps, first);
+int ns2d_tlrec_run(Ctx *c, int nsteps, bool first, bool last) {
+  return c->rec_p == 4 ? run2tlrec_t<float>(c, nsteps, first, last) : run2tlrec_t<double>(c, nsteps, first, last);
 }
 
 int ns2d_rec_reset(Ctx *c) {

@@ -389,10 +389,11 @@ int ns3d_work_end(Ctx *c) {
   return work_copy<double, double, false>(c, c->stw, c->state);
 }
 
-int ns3d_run(Ctx *c, int nsteps, bool first) {
+int ns3d_run(Ctx *c, int nsteps, bool first, bool last) {
   const bool own = !c->work_live;
   if (own) PSG_TRY(ns3d_work_begin(c));
-  const int r = c->wsplit ? (c->st32 ? split_run<float>(c, c->st32, nsteps, first) : split_run<double>(c, c->stw, nsteps, first))
+  const int r = c->wsplit ? (c->st32 ? split_run<float>(c, c->st32, nsteps, first, last)
+                                     : split_run<double>(c, c->stw, nsteps, first, last))
                           : (c->st32 ? run_t<float, float>(c, c->st32, nsteps, first)
                                      : run_t<double, double>(c, c->stw, nsteps, first));
   if (!own) return r;

@@ -2,5 +2,5 @@
 #include "psg_split.hpp"
 
 namespace psg {
-template int split_run<float>(Ctx *, cpx<float> *, int, bool);
+template int split_run<float>(Ctx *, cpx<float> *, int, bool, bool);
 }  // namespace psg

@@ -2,5 +2,5 @@
 #include "psg_split.hpp"
 
 namespace psg {
-template int split_run<double>(Ctx *, cpx<double> *, int, bool);
+template int split_run<double>(Ctx *, cpx<double> *, int, bool, bool);
 }  // namespace psg
