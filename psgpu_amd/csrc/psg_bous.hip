@@ -25,8 +25,9 @@ typedef LayRun<12> LayXS;
 // seventh field is rho itself (physical-space dumps, 3D_Boussinesq/src/out_low.h:79-110)
 // LAY: layout of st (its field stride fs); the mask is in the reference order.
 // Gather- and register-bound: vorticity becomes velocity in its own registers,
-// in FP64 until the transforms, and every index is a constant, so that nothing
-// of a pencil lies in scratch memory and two waves share a SIMD (an earlier
+// in FP64 until the transforms, and every index is a constant, so that with whole
+// pencils of up to 512 points nothing lies in scratch memory and two waves share a
+// SIMD (split fields in FP64 keep up to 52 bytes there, 1024 points 232 to 472; an earlier
 // form, with the field loop rolled, indexed its registers at run time: 400 bytes
 // of scratch a lane and one wave per SIMD; capped for three waves this one spills
 // and is slower again).  512^3 FP64 2.11 -> 1.54 ms, 256^3 0.289 -> 0.195 ms, in
@@ -311,8 +312,12 @@ template <typename P> static int xpass_bous(Ctx *c, const cpx<P> *B, cpx<P> *Cb,
   //   FP64, 256 points on: 3 (8 points a thread 516, this 394 at 256^3; 4530, 3543 at 512^3), 32 to 128: 4
   //     (16.8, 14.2 at 32^3; 17.9, 15.0 at 64^3; 70.0, 60.3 at 128^3; 117, 98.8 at 64^3 with 16 members)
   //   FP32, 32 and 64: 4 (15.8, 12.8; 15.1, 13.0), 128: 2 (37.2, 35.6), above: 8 points, product kept
-  //   16 points: 4 is faster too (19.1, 10.8), but the radix stays 8: its rounding decides
-  //     where a Newton iteration with a singular Jacobian stops on these smallest grids
+  //   16 points: 8 points a thread although 4 is faster (19.1, 10.8).  This is not a matter of
+  //     speed or of accuracy: a two-shift Newton solve at 16^3 whose Jacobian is singular stops
+  //     at a shift of 1.34e-5 with the radix-4 shapes (3, 4, 7, 8, 9, 11) and below 1e-5, the
+  //     bound that is asked of it, with the radix-8 ones
+  // Shape 3 and 4 add in another order (radix 4 throughout): one 512^3 step is 1.8e-16 of its
+  // state off its 64-bit value, and 1.6e-16 with radix 8
   const int n = c->g.nx;
   const int best = n < 32 ? 0 : sizeof(P) == 8 ? (n >= 256 ? 3 : 4) : (n <= 64 ? 4 : n == 128 ? 2 : 0);
   const int xv = c->xvar ? c->xvar : best;
@@ -349,7 +354,9 @@ template <typename P, class UPD> static int launch_zfwd_b(Ctx *c, const cpx<P> *
     // registers (up to 290 in FP64, one wave per SIMD).  From 256 points on there
     // are blocks enough for occupancy to count: the update's loads stay within
     // pairs of modes, and in FP64 each field is loaded at its own transform
-    // (256^3 FP64 297 -> 229 us, FP32 209 -> 201; at 64^3 it would be 21 -> 26)
+    // (256^3 FP64 297 -> 229 us, FP32 209 -> 201; at 64^3 it would be 21 -> 26).  Two
+    // waves per SIMD leave 256 registers a thread: FP64 keeps 104 to 200 bytes a lane
+    // in scratch, FP32 none.  Either way it waits for memory for 61 to 81% of its time
     constexpr bool LONG = N >= 256;
     auto k = k_zfwd<P, N, T, 4, UPD, (sizeof(P) == 4 || !LONG), 1, (LONG ? 2 : 0), (LONG && N <= 512 ? 2 : 1)>;
     PSG_HIP(lds_attr(k, lds));

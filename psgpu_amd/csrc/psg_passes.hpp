@@ -203,7 +203,10 @@ template <typename P> __device__ __forceinline__ long yoff(const Grid &g, int ik
 //  YCol : 2D, one kx column after the other ([ikx][y]), for the products too: a
 //         2D column pass owns single columns and reads and writes each as one
 //         run; the x-pass gathers its row from lines that it shares with the
-//         seven rows beside it, which xcd_tile puts on the same XCD
+//         rows beside it (8 of a line in FP64, 16 in FP32), which xcd_tile puts
+//         on the same XCD.  The pitch is 8 points more than the column: columns
+//         start an odd number of 128-byte lines apart in FP64, of 64-byte halves
+//         in FP32, so that the elements of a row spread over the L2 channels
 template <typename P> struct YTile {
   static __device__ __forceinline__ long row(const Grid &g, int y, int z) { return yoff<P>(g, 0, y, z); }
   static __device__ __forceinline__ int col(const Grid &g, int k) {
@@ -211,8 +214,6 @@ template <typename P> struct YTile {
     return (k >> SH) * (g.ny * W) + (k & (W - 1));
   }
 };
-//         (pitch: columns start an odd number of 128-byte lines apart, so that
-//         the elements of a row spread over the L2 channels)
 struct YCol {
   static __host__ __device__ __forceinline__ int pitch(const Grid &g) { return g.ny + 8; }
   static __device__ __forceinline__ long row(const Grid &, int y, int) { return y; }

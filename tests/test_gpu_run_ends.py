@@ -64,3 +64,23 @@ def test_tangents_of_any_length(gpu, graph, prec, tol):
             assert np.abs(z1 - zf).max() <= tol * np.abs(zf).max(), T
             assert np.abs(z2 - zf).max() <= tol * np.abs(zf).max(), T
             assert np.abs(d2 - d1).max() <= 2 * tol * np.abs(d1).max(), T
+
+
+@pytest.mark.parametrize("nx,ny", [(16, 16), (32, 64), (64, 32), (128, 128), (256, 256), (64, 512), (32, 1024)])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_captured_steps_at_the_end_give_the_bits_of_direct_launches(gpu, nx, ny, prec):
+    # the last stage of direct launches only updates, that of captured steps also transforms
+    g = O.grid2(nx, ny, ny / nx)
+    z, d = O.ic_ns2d_cfg(g, 5, 1.0), O.ic_ns2d_cfg(g, 6, 1.0)
+    with P.Stepper(flavour="ns2d", nx=nx, ny=ny, n=ny, alpha=ny / nx, v2=1 / 40, dt=0.005, kf=4.0, ampfor=-2.0,
+                   precision=prec) as s:
+        out = []
+        for graph in (0, 4):
+            s.set_graph(graph)
+            s.set_dt(0.005)   # the tangents leave their own
+            s.set_state(z[None])
+            s.run(9)
+            out.append((s.get_state(),) + s.tangent(z[None], d[None], 9.5 * 0.005, 0.005)
+                       + s.tangent_many(z[None], d[None, None], 9.5 * 0.005, 0.005))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
